@@ -8,8 +8,8 @@
 //   Q  lpos 0 only, b < 144: LN1 + QKV of the block input (the global hidden
 //      state), RoPE, k/v into the local cache                  -> LL q|k|v
 //   A  b < 12: head h = b: the step's input -- for lpos >= 2 the code of the
-//      previous channel, picked here (greedy: penalised argmax of its logits,
-//      or the forced code) or written by the sampler -- and the head's q|k|v:
+//      previous channel, picked here (penalised argmax of its logits, or a draw
+//      from them, or the forced code) -- and the head's q|k|v:
 //      from the QKV stage (lpos 0) or from the precomputed row of (lpos,
 //      code); k/v into the local cache; the head's attention over keys
 //      0..lpos (at most 17)                                    -> LL attn + code
@@ -29,6 +29,7 @@
 #include "mh_gemv.h"
 #include "mh_ll.h"
 #include "mh_ops.h"
+#include "mh_sample.h"
 
 namespace mh {
 namespace {
@@ -41,7 +42,8 @@ constexpr int kLH = kLX + kHidden;      // fc_in output
 constexpr int kLO = kLH + kFF;          // block output (head input)
 constexpr int kLL = kLO + kHidden;      // head logits, the next step's pick input (1024)
 constexpr int kLG = kLL + kCodebook;    // position 0's block output, the end gate's input (768)
-static_assert(kLG + kHidden <= kLayerWords, "local LL layout fits the exchange buffer");
+constexpr int kLD = kLG + kHidden;      // sampled frames: the end gate is done (1)
+static_assert(kLD + 1 <= kLayerWords, "local LL layout fits the exchange buffer");
 
 // Stage timestamps (100 MHz device clock) of the last launch, per workgroup,
 // in builds with -DMH_STAGE_TRACE only.
@@ -79,8 +81,19 @@ namespace {
     } while (0)
 #endif
 
+template <bool SAMPLED>
+__device__ __forceinline__ SampleLds &sample_lds() {  // in LDS only where a kernel draws
+    __shared__ SampleLds l;
+    return l;
+}
+
 // A8: every GEMV in W8A8 (quant_act_lds), the reference's decode with MOSS_A16 unset.
-template <bool A8>
+// SAMPLED: the frame draws its codes (sampler.cpp:30-78) unless it is one of the call's greedy
+// first frames.  Each of the 12 attention workgroups makes the same draw from its own copy of
+// the call's xoshiro stream, so a pick costs its ~4 us of sorting and no hand-off; one launch
+// per position with a sampler kernel after each measured 0.88 ms per frame's local half
+// (17 x 16 us + 16 x 38 us, W8A8).
+template <bool A8, bool SAMPLED>
 __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
 #pragma clang fp contract(off)
     __shared__ float act[kFF + 1];
@@ -91,9 +104,9 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
     __shared__ float part[4][4];
     __shared__ float pbv[4];
     __shared__ int pbi[4];
-    __shared__ int used_s;
     __shared__ float lgt[kCodebook];  // the previous step's logits (chained launches)
     __shared__ GateLds gl;
+    SampleLds &sl = sample_lds<SAMPLED>();
 
     __shared__ int wait_failed;  // set when a wait of this workgroup runs out
     if (threadIdx.x == 0) wait_failed = 0;
@@ -105,6 +118,17 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
     const uint32_t tag_base = (uint32_t)(st->pos + 1) << 5;
     int budget = a.poll_budget > 0 ? a.poll_budget : kPollBudget;
     uint64_t *LL = a.ll;
+    // SAMPLED: this frame's stream.  The end gate draws first (llm.cpp:678) when it samples at all;
+    // workgroup 0 stores the state after the frame's last draw.
+    bool draws = false;
+    uint32_t rng[4], gate_rng[4];
+    if constexpr (SAMPLED) {
+        const SampleCfg c = st->cfg;
+        draws = !c.greedy && st->frame >= c.greedy_frames;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gate_rng[i] = rng[i] = st->rng[i];
+        if (!c.end_greedy && st->frame >= st->min_frames) (void)rng_next(rng);
+    }
 
     // ---- the end gate (llm.cpp:653-679) in a workgroup of its own (the last):
     // ln_f of position 0's block output, the 2-row W8A8 gate, the stop rule.  The
@@ -128,9 +152,19 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
 #pragma unroll
         for (int i = 0; i < 3; ++i) act[t + 256 * i] = o[i];
         __syncthreads();
-        gate_block(act, a.wte, st, gl);
+        gate_block(act, a.wte, st, gl, SAMPLED ? gate_rng : st->rng);
+        // workgroup 0 changes the frame number and the stream only after the gate has read them
+        if constexpr (SAMPLED)
+            if (t == 0) ll_put(LL + kLD, 1.0f, tag_base | 12u);
         return;
     }
+
+    auto pick = [&](const PickIn &in) {  // by every thread of the workgroup, the same in all of them
+        if constexpr (SAMPLED)
+            if (draws) return pick_penalised(in, st->rep_penalty, st->cfg, rng_uniform(rng), sl);
+        const int idx = greedy_pick_reduce(in, st->rep_penalty, pbv, pbi);
+        return idx >= kCodebook ? 0 : idx;  // every value NaN: the reference's scan stays at 0
+    };
 
 #pragma unroll 1
     for (int lpos = a.lpos; lpos <= a.lpos_last; ++lpos) {
@@ -144,8 +178,7 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
         const uint8_t *head_w = a.head && lpos >= 1 ? a.aemb[lpos - 1] : nullptr;
         float *logits_out = lpos >= 1 ? a.logits + (size_t)(lpos - 1) * kCodebook : nullptr;
         const bool live = lpos == 0;  // the block input is the global hidden state: QKV computed here
-        const bool picking = !live && ch_in >= 0 && a.pick;
-        const bool pick_ll = picking && lpos > a.lpos;  // logits from this launch's previous step
+        const bool picking = !live && ch_in >= 0;  // from the previous step's logits
         // W8A8 quantiser capture of this position (tests only; null in the library's own use)
         float *const cap = A8 && a.cap ? a.cap + (size_t)lpos * MOSS_HIP_CAP_STEP : nullptr;
 
@@ -201,16 +234,10 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
             const int kmax = max(lpos - 1, 0);
             // loads complete in issue order: the pick's logits first
             PickIn pin;
-            if (picking) {
-                if (pick_ll) {  // counts now, values once the previous step's head has stored them
+            if (picking)  // counts now, values once the previous step's head has stored them
 #pragma unroll
-                    for (int k = 0; k < kCodebook / 256; ++k)
-                        pin.cnt[k] = st->rep_penalty != 1.0f ? a.counts[(size_t)ch_in * kCodebook + t + 256 * k] : 0;
-                } else {
-                    greedy_pick_load(a.logits + (size_t)ch_in * kCodebook, a.counts + (size_t)ch_in * kCodebook,
-                                     st->rep_penalty, pin);
-                }
-            }
+                for (int k = 0; k < kCodebook / 256; ++k)
+                    pin.cnt[k] = st->rep_penalty != 1.0f ? a.counts[(size_t)ch_in * kCodebook + t + 256 * k] : 0;
             // the cache rows (keys 0 .. lpos-1, written by earlier launches) before
             // anything else; the key at lpos, and the clamped ones past it, take
             // this step's row below
@@ -237,34 +264,23 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
                 }
             } else {
                 const float *row = a.qkv_table;  // lpos 1: wte[slot]
-                if (ch_in >= 0) {
-                    int used;
-                    if (picking) {  // greedy pick of channel ch_in (llm.cpp:689-697)
-                        if (pick_ll) {
-                            // waves 1-3 poll the logits: wave 0's cache-row loads, issued
-                            // above, would hold back its polls (loads complete in order)
-                            bool ok = true;
-                            if (t >= 64)
-                                ok = ll_gather_by<(kCodebook + 191) / 192, 192>(LL + kLL, kCodebook, tag - 1, lgt,
-                                                                                 budget, t - 64);
-                            if (sync_failed(!ok, &wait_failed)) {
-                                if (t == 0) atomicOr(a.err, 1u);
-                                return;
-                            }
+                if (picking) {  // the pick of channel ch_in (llm.cpp:689-697)
+                    // waves 1-3 poll the logits: wave 0's cache-row loads, issued
+                    // above, would hold back its polls (loads complete in order)
+                    bool ok = true;
+                    if (t >= 64)
+                        ok = ll_gather_by<(kCodebook + 191) / 192, 192>(LL + kLL, kCodebook, tag - 1, lgt, budget, t - 64);
+                    if (sync_failed(!ok, &wait_failed)) {
+                        if (t == 0) atomicOr(a.err, 1u);
+                        return;
+                    }
 #pragma unroll
-                            for (int k = 0; k < kCodebook / 256; ++k) pin.vals[k] = lgt[t + 256 * k];
-                        }
-                        int idx = greedy_pick_reduce(pin, st->rep_penalty, pbv, pbi);
-                        if (idx >= kCodebook) idx = 0;
-                        used = st->forced_on ? a.forced[st->frame * kNVq + ch_in] : idx;
-                        if (b == 0 && t == 0) {
-                            st->codes[ch_in] = idx;
-                            st->row[ch_in + 1] = used;
-                        }
-                    } else {  // written by the sampler of channel ch_in
-                        if (t == 0) used_s = st->row[ch_in + 1];
-                        __syncthreads();
-                        used = used_s;
+                    for (int k = 0; k < kCodebook / 256; ++k) pin.vals[k] = lgt[t + 256 * k];
+                    const int idx = pick(pin);
+                    const int used = st->forced_on ? a.forced[st->frame * kNVq + ch_in] : idx;
+                    if (b == 0 && t == 0) {
+                        st->codes[ch_in] = idx;
+                        st->row[ch_in + 1] = used;
                     }
                     if (b == 0 && t == 0) ll_put(LL + kLA + kHidden, __int_as_float(used), tag);  // for stage P
                     row = a.qkv_table + (1 + (size_t)ch_in * kCodebook + used) * 3 * kHidden;
@@ -501,7 +517,7 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
             STAGE_TS(10);
         }
 
-        // ---- after the last position: the greedy pick of its channel, as
+        // ---- after the last position: the pick of its channel, as
         // sample_kernel does for the last channel (workgroup 0)
         if (a.final_pick && lpos == a.lpos_last && b == 0) {
             const int ch = lpos - 1;
@@ -509,15 +525,15 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
 #pragma unroll
             for (int k = 0; k < kCodebook / 256; ++k)
                 pin.cnt[k] = st->rep_penalty != 1.0f ? a.counts[(size_t)ch * kCodebook + t + 256 * k] : 0;
-            const bool ok = ll_gather<kCodebook / 256>(LL + kLL, kCodebook, tag, lgt, budget);
+            bool ok = ll_gather<kCodebook / 256>(LL + kLL, kCodebook, tag, lgt, budget);
+            if constexpr (SAMPLED) ok = ll_wait1(LL + kLD, t == 0 && a.gate, tag_base | 12u, &pbv[0], budget) && ok;
             if (sync_failed(!ok, &wait_failed)) {
                 if (t == 0) atomicOr(a.err, 1u);
                 return;
             }
 #pragma unroll
             for (int k = 0; k < kCodebook / 256; ++k) pin.vals[k] = lgt[t + 256 * k];
-            int idx = greedy_pick_reduce(pin, st->rep_penalty, pbv, pbi);
-            if (idx >= kCodebook) idx = 0;
+            const int idx = pick(pin);
             const int used = st->forced_on ? a.forced[st->frame * kNVq + ch] : idx;
             if (t < ch) a.counts[(size_t)t * kCodebook + st->row[t + 1]] += 1;  // the frame's earlier channels
             if (t == 0) {
@@ -526,6 +542,9 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
                 a.counts[(size_t)ch * kCodebook + used] += 1;
                 st->row[0] = kSlotToken;
                 st->frame += 1;
+                if constexpr (SAMPLED)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) st->rng[i] = rng[i];
             }
         }
     }  // lpos
@@ -542,12 +561,15 @@ extern "C" int mh_local_trace_read(unsigned long long *out) {
 #endif
 
 hipError_t decode_local_occupancy(int *per_cu) {
-    int p16 = 0, p8 = 0;
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&p16, decode_local_kernel<false>, 256, 0);
-    if (e != hipSuccess) return e;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&p8, decode_local_kernel<true>, 256, 0);
-    *per_cu = p16 < p8 ? p16 : p8;
-    return e;
+    const void *k[4] = {(const void *)decode_local_kernel<false, false>, (const void *)decode_local_kernel<true, false>,
+                        (const void *)decode_local_kernel<false, true>, (const void *)decode_local_kernel<true, true>};
+    for (int i = 0; i < 4; ++i) {
+        int p = 0;
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, k[i], 256, 0);
+        if (e != hipSuccess) return e;
+        *per_cu = i == 0 || p < *per_cu ? p : *per_cu;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_decode_local(const LocalArgs &a, hipStream_t s) {
@@ -562,15 +584,19 @@ hipError_t launch_decode_local(const LocalArgs &a, hipStream_t s) {
     if (a.gate && (a.lpos != 0 || !a.wte || !a.lnf_w || !a.lnf_b)) return hipErrorInvalidValue;
     if (a.lpos_last >= 1 && !a.qkv_table) return hipErrorInvalidValue;
     if (a.lpos <= 1 && a.lpos_last >= 1 && !a.x_slot) return hipErrorInvalidValue;
-    if (a.lpos_last >= 2 && a.pick && (!a.logits || !a.counts || !a.forced)) return hipErrorInvalidValue;
-    // a chained pick reads the previous step's head: every step but the last runs one
-    if (a.lpos_last > a.lpos && a.lpos_last >= 2 && a.pick && !a.head) return hipErrorInvalidValue;
-    if (a.final_pick && (!a.pick || !a.head || a.lpos_last < 1 || !a.counts || !a.forced)) return hipErrorInvalidValue;
+    // a pick reads the logits of the launch's previous step: the steps run as one chain with heads
+    if (a.lpos_last >= 2 && (a.lpos > 1 || !a.head || !a.counts || !a.forced)) return hipErrorInvalidValue;
+    if (a.final_pick && (!a.head || a.lpos_last < 1 || !a.counts || !a.forced)) return hipErrorInvalidValue;
     // one more workgroup for the end gate
-    if (a.a8)
-        hipLaunchKernelGGL(decode_local_kernel<true>, dim3(kLayerGrid + (a.gate ? 1 : 0)), dim3(256), 0, s, a);
+    const dim3 grid(kLayerGrid + (a.gate ? 1 : 0));
+    if (a.a8 && a.sampled)
+        hipLaunchKernelGGL((decode_local_kernel<true, true>), grid, dim3(256), 0, s, a);
+    else if (a.a8)
+        hipLaunchKernelGGL((decode_local_kernel<true, false>), grid, dim3(256), 0, s, a);
+    else if (a.sampled)
+        hipLaunchKernelGGL((decode_local_kernel<false, true>), grid, dim3(256), 0, s, a);
     else
-        hipLaunchKernelGGL(decode_local_kernel<false>, dim3(kLayerGrid + (a.gate ? 1 : 0)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((decode_local_kernel<false, false>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -1,5 +1,6 @@
 // frame_ops.hip -- the small per-step kernels around the GEMVs (gfx950).
 #include "mh_ops.h"
+#include "mh_sample.h"
 
 namespace mh {
 namespace {
@@ -54,146 +55,6 @@ __global__ __launch_bounds__(256) void dequant_rows_kernel(const uint8_t *w, int
         out[(size_t)blockIdx.x * cols + c] = ok ? q8x4_elem(w, nb, r, c) : __int_as_float(0x7fc00000);
 }
 
-// ---- sample_token (reference csrc/src/sampler.cpp:9-79) for one 1024-entry
-// logit row, by one 256-thread workgroup.  The caller has applied the
-// repetition penalty into vals[] (LDS).
-
-struct PickLds {
-    float vals[kCodebook];     // penalised (then temperature-scaled) logits
-    uint64_t keys[kCodebook];  // sort keys: value descending, index ascending
-    float ex[kCodebook];       // exp(v - max) of the candidates, in sorted order
-    float bv[4];
-    int bi[4];
-    int pick;
-    int used;
-};
-
-// Greedy branch (sampler.cpp:23-28): argmax, the lowest index wins ties, NaN values
-// never win; index 0 when the value at index 0 is NaN or every value is NaN (the
-// reference's scan compares with its best so far, so it never moves off a NaN at 0).
-__device__ int pick_greedy(PickLds &L) {
-    const int t = threadIdx.x;
-    float best = -INFINITY;
-    int besti = kCodebook;
-    for (int i = t; i < kCodebook; i += 256) {  // ascending i per thread
-        const float v = L.vals[i];
-        if (v > best) {
-            best = v;
-            besti = i;
-        }
-    }
-    wave_argmax(best, besti);
-    if ((t & 63) == 0) {
-        L.bv[t >> 6] = best;
-        L.bi[t >> 6] = besti;
-    }
-    __syncthreads();
-    if (t == 0) {
-        float b = L.bv[0];
-        int idx = L.bi[0];
-        for (int w = 1; w < 4; ++w)
-            if (L.bv[w] > b || (L.bv[w] == b && L.bi[w] < idx)) {
-                b = L.bv[w];
-                idx = L.bi[w];
-            }
-        L.pick = (idx >= kCodebook || L.vals[0] != L.vals[0]) ? 0 : idx;
-    }
-    __syncthreads();
-    return L.pick;
-}
-
-// Order-preserving map of a float to uint32 (larger float -> larger key).
-__device__ __forceinline__ uint32_t float_order(float f) {
-    const uint32_t u = __float_as_uint(f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-
-// Sampling branch (sampler.cpp:30-78): temperature, top-k by a full sort
-// (value descending; equal values by index), softmax over the k candidates,
-// top-p cut, one uniform draw walked down the sorted candidates.  The
-// sequential sums run in one thread in the reference's order.
-__device__ int pick_sampled(PickLds &L, const SampleCfg &c, uint32_t *rng) {
-#pragma clang fp contract(off)
-    const int t = threadIdx.x;
-    const bool scale = c.temperature > 0.0f && c.temperature != 1.0f;
-    const float inv = scale ? 1.0f / c.temperature : 1.0f;
-    for (int i = t; i < kCodebook; i += 256) {
-        float v = L.vals[i];
-        if (scale) v = v * inv;
-        L.vals[i] = v;
-        L.keys[i] = ((uint64_t)(~float_order(v)) << 32) | (uint32_t)i;
-    }
-    __syncthreads();
-    // bitonic sort, ascending keys
-    for (int k = 2; k <= kCodebook; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = t; i < kCodebook; i += 256) {
-                const int ixj = i ^ j;
-                if (ixj > i) {
-                    const uint64_t a = L.keys[i], b = L.keys[ixj];
-                    const bool up = (i & k) == 0;
-                    if ((a > b) == up) {
-                        L.keys[i] = b;
-                        L.keys[ixj] = a;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-    const int n = c.top_k > 0 ? (c.top_k < kCodebook ? c.top_k : kCodebook) : kCodebook;
-    const float maxv = L.vals[(int)(L.keys[0] & 0xffffffffu)];
-    for (int i = t; i < n; i += 256) L.ex[i] = expf(L.vals[(int)(L.keys[i] & 0xffffffffu)] - maxv);
-    __syncthreads();
-    if (t == 0) {
-        float sum = 0.0f;
-        for (int i = 0; i < n; ++i) sum += L.ex[i];
-        int cnt = n;
-        if (c.top_p < 1.0f) {
-            float cum = 0.0f;
-            int keep = 0;
-            for (; keep < n; ++keep) {
-                cum += L.ex[keep] / sum;
-                if (cum >= c.top_p) {
-                    ++keep;
-                    break;
-                }
-            }
-            cnt = keep > 1 ? keep : 1;
-            sum = 0.0f;
-            for (int i = 0; i < cnt; ++i) sum += L.ex[i];
-        }
-        float r = rng_uniform(rng) * sum;
-        int pick = (int)(L.keys[cnt - 1] & 0xffffffffu);
-        for (int i = 0; i < cnt; ++i) {
-            r -= L.ex[i];
-            if (r <= 0.0f) {
-                pick = (int)(L.keys[i] & 0xffffffffu);
-                break;
-            }
-        }
-        L.pick = pick;
-    }
-    __syncthreads();
-    return L.pick;
-}
-
-// vals[i] = logits[i] with the repetition penalty applied once per past
-// occurrence of i (sampler.cpp:13-21: v<0 ? v*p : v/p, repeated).  Each index
-// is penalised independently, so per-index counts reproduce the reference's
-// walk over the history exactly.
-__device__ void load_penalised(PickLds &L, const float *logits, const int *counts, float p) {
-#pragma clang fp contract(off)
-    for (int i = threadIdx.x; i < kCodebook; i += 256) {
-        float v = logits[i];
-        if (p != 1.0f) {
-            const int c = counts[i];
-            for (int k = 0; k < c; ++k) v = v < 0.0f ? v * p : v / p;
-        }
-        L.vals[i] = v;
-    }
-    __syncthreads();
-}
-
 // End gate (reference csrc/src/llm.cpp:274-285 + :30-35 + :678):
 //  1. h = LayerNorm(x; local lnf)                     (the local step's output)
 //  2. W8A8 quantisation of h per 32-block            (csrc/src/quant.cpp:28-43):
@@ -221,7 +82,7 @@ __global__ __launch_bounds__(256) void gate_kernel(const float *x_raw, const flo
 #pragma unroll
     for (int i = 0; i < 3; ++i) hbuf[t + 256 * i] = o[i];
     __syncthreads();
-    gate_block(hbuf, wte, state, g);
+    gate_block(hbuf, wte, state, g, state->rng);
 }
 
 // End gate of a frame whose gate is dumped (llm.cpp:653-679): the reference then
@@ -276,29 +137,42 @@ __global__ __launch_bounds__(256) void gate_text_kernel(const float *logits, Dev
 // teacher forcing) is counted into the history, written into the next
 // global-step row, and its aemb row becomes the next local input.
 __global__ __launch_bounds__(256) void sample_kernel(SampleArgs a) {
-    __shared__ PickLds L;
+    __shared__ SampleLds L;
+    __shared__ float bv[4];
+    __shared__ int bi[4], used_s;
     DevState *st = a.state;
     const bool stopped = st->stop;  // tested once the logits are loaded
     const int t = threadIdx.x;
-    load_penalised(L, a.logits, a.counts + a.ch * kCodebook, st->rep_penalty);
+    const float pen = st->rep_penalty;
+    PickIn in;
+    greedy_pick_load(a.logits, a.counts + a.ch * kCodebook, pen, in);
     if (stopped) return;
     const SampleCfg c = st->cfg;
     const bool greedy = c.greedy || st->frame < c.greedy_frames;
-    const int idx = greedy ? pick_greedy(L) : pick_sampled(L, c, st->rng);
+    uint32_t rng[4] = {st->rng[0], st->rng[1], st->rng[2], st->rng[3]};
+    int idx;
+    if (greedy) {
+        idx = greedy_pick_reduce(in, pen, bv, bi);
+        idx = idx >= kCodebook ? 0 : idx;  // every value NaN: the reference's scan stays at 0
+    } else {
+        idx = pick_penalised(in, pen, c, rng_uniform(rng), L);
+    }
     if (a.count_all && t < a.ch) a.counts[t * kCodebook + st->row[t + 1]] += 1;  // one channel per thread
     if (t == 0) {
         const int used = st->forced_on ? a.forced[st->frame * kNVq + a.ch] : idx;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) st->rng[i] = rng[i];
         st->codes[a.ch] = idx;
         st->row[a.ch + 1] = used;
         a.counts[a.ch * kCodebook + used] += 1;
-        L.used = used;
+        used_s = used;
         if (a.last_channel) {
             st->row[0] = kSlotToken;
             st->frame += 1;
         }
     }
     __syncthreads();
-    const int used = L.used;
+    const int used = used_s;
     const int nb = kHidden / 32;
     for (int c2 = t; c2 < kHidden; c2 += 256) a.next_input[c2] = q8x4_elem(a.aemb, nb, used, c2);
 }
@@ -602,7 +476,9 @@ __global__ __launch_bounds__(256) void local_qkv_rows_kernel(LocalQkv a) { local
 __global__ __launch_bounds__(256) void sample_rows_kernel(const float *logits, int ch, const uint8_t *aemb,
                                                           float *next_in, StreamState st, int last_channel,
                                                           LocalQkv next, int count_prev) {
-    __shared__ PickLds L;
+    __shared__ SampleLds L;
+    __shared__ float bv[4];
+    __shared__ int bi[4];
     const int srow = blockIdx.x, t = threadIdx.x;
     float *nxt = next_in + (size_t)srow * kHidden;
     const int nb = kHidden / 32;
@@ -626,11 +502,19 @@ __global__ __launch_bounds__(256) void sample_rows_kernel(const float *logits, i
             if (pen == 1.0f)
 #pragma unroll
                 for (int k = 0; k < kCodebook / 256; ++k) in.cnt[k] = 0;
-            idx = greedy_pick_reduce(in, pen, L.bv, L.bi);
+            idx = greedy_pick_reduce(in, pen, bv, bi);
             idx = idx >= kCodebook ? 0 : idx;  // every value NaN: the reference's scan stays at 0
         } else {
-            load_penalised(L, lg, cnt, pen);
-            idx = pick_sampled(L, c, st.rng + 4 * srow);
+            if (pen == 1.0f)
+#pragma unroll
+                for (int k = 0; k < kCodebook / 256; ++k) in.cnt[k] = 0;
+            uint32_t rng[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) rng[i] = st.rng[4 * srow + i];
+            idx = pick_penalised(in, pen, c, rng_uniform(rng), L);  // (a barrier inside: every thread has read rng)
+            if (t == 0)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) st.rng[4 * srow + i] = rng[i];
         }
         if (t == 0) {
             st.codes[srow * kNVq + ch] = idx;

@@ -453,63 +453,37 @@ void Model::enqueue_local_step(hipStream_t s, const float *in, int lpos, int pic
 // channel ch's QKV GEMV instead of a kernel of its own; only channel 15 keeps
 // its sample kernel, which also counts the frame's used codes.
 void Model::enqueue_frame_local(hipStream_t s, bool text_gate, bool fused) {
-    if (fused_layers_ && !text_gate) {  // one launch when greedy; else per position with a sampler between
-        LocalArgs base;
+    if (fused_layers_ && !text_gate) {  // one launch
+        LocalArgs c;
         const LayerW &L = local_;
-        base.attn_w = L.attn_w; base.proj_w = L.proj_w; base.fc_in_w = L.fc_in_w; base.fc_out_w = L.fc_out_w;
-        base.attn_b = L.attn_b; base.proj_b = L.proj_b; base.fc_in_b = L.fc_in_b; base.fc_out_b = L.fc_out_b;
-        base.ln1_w = L.ln1_w; base.ln1_b = L.ln1_b; base.ln2_w = L.ln2_w; base.ln2_b = L.ln2_b;
-        base.lnf_w = llnf_w_; base.lnf_b = llnf_b_;
-        base.lk = lkv_; base.lv = lkv_ + (size_t)kHeads * kLocalLen * kHeadDim;
-        base.rope_cos = rope_; base.rope_sin = rope_ + (size_t)rope_n_ * kRopeHalf;
-        base.state = state_; base.ll = ll_; base.err = &state_->ll_err; base.x_out = lres_;
-        base.a8 = decode_a8_;
-        base.poll_budget = next_poll_budget();
+        c.attn_w = L.attn_w; c.proj_w = L.proj_w; c.fc_in_w = L.fc_in_w; c.fc_out_w = L.fc_out_w;
+        c.attn_b = L.attn_b; c.proj_b = L.proj_b; c.fc_in_b = L.fc_in_b; c.fc_out_b = L.fc_out_b;
+        c.ln1_w = L.ln1_w; c.ln1_b = L.ln1_b; c.ln2_w = L.ln2_w; c.ln2_b = L.ln2_b;
+        c.lnf_w = llnf_w_; c.lnf_b = llnf_b_;
+        c.lk = lkv_; c.lv = lkv_ + (size_t)kHeads * kLocalLen * kHeadDim;
+        c.rope_cos = rope_; c.rope_sin = rope_ + (size_t)rope_n_ * kRopeHalf;
+        c.state = state_; c.ll = ll_; c.err = &state_->ll_err; c.x_out = lres_;
+        c.a8 = decode_a8_;
+        c.poll_budget = next_poll_budget();
         if (capture_ && decode_a8_) {
-            base.cap = cap_dec_ + (size_t)kLayers * MOSS_HIP_CAP_STEP;
+            c.cap = cap_dec_ + (size_t)kLayers * MOSS_HIP_CAP_STEP;
             cap_taken_[1] = true;
         }
-        for (int ch = 0; ch < kNVq; ++ch) base.aemb[ch] = aemb_[ch];
-        base.qkv_table = qkv_table_;
-        base.logits = logits_;
-        base.counts = counts_;
-        base.forced = forced_;
-        base.x_in = hidden_;
-        base.x_slot = slot_in_;
-        if (fused) {  // greedy: the whole local half in one launch (positions 0..16, the gate, channel 15's pick)
-            LocalArgs c = base;
-            c.lpos = 0;
-            c.lpos_last = kNVq;
-            c.head = 1;
-            c.pick = 1;
-            c.gate = 1;
-            c.wte = wte_;
-            c.final_pick = 1;
-            hip_check(launch_decode_local(c, s), "local steps");
-            return;
-        }
-        LocalArgs z = base;  // lpos 0 on the global hidden state, then the end gate
-        z.lpos = 0;
-        z.lpos_last = 0;
-        hip_check(launch_decode_local(z, s), "local step");
-        hip_check(launch_gate(lres_, llnf_w_, llnf_b_, wte_, state_, s), "gate");
-        LocalArgs c = base;  // the channel steps: input wte[slot] at lpos 1, then aemb[ch - 1][code]
+        for (int ch = 0; ch < kNVq; ++ch) c.aemb[ch] = aemb_[ch];
+        c.qkv_table = qkv_table_;
+        c.logits = logits_;
+        c.counts = counts_;
+        c.forced = forced_;
+        c.x_in = hidden_;
+        c.x_slot = slot_in_;
+        c.lpos = 0;  // positions 0..16, the gate and every channel's pick
+        c.lpos_last = kNVq;
         c.head = 1;
-        SampleArgs sa;
-        sa.counts = counts_;
-        sa.forced = forced_;
-        sa.next_input = next_in_;
-        sa.state = state_;
-        for (int ch = 0; ch < kNVq; ++ch) {
-            c.lpos = c.lpos_last = ch + 1;
-            hip_check(launch_decode_local(c, s), "local step");
-            sa.logits = logits_ + (size_t)ch * kCodebook;
-            sa.ch = ch;
-            sa.aemb = aemb_[ch];
-            sa.last_channel = ch == kNVq - 1;
-            sa.count_all = 0;
-            hip_check(launch_sample(sa, s), "sample");
-        }
+        c.gate = 1;
+        c.wte = wte_;
+        c.final_pick = 1;
+        c.sampled = fused ? 0 : 1;
+        hip_check(launch_decode_local(c, s), "local steps");
         return;
     }
     enqueue_local_step(s, hidden_, 0, -1);
@@ -545,23 +519,19 @@ void Model::enqueue_frame_local(hipStream_t s, bool text_gate, bool fused) {
 }
 
 // Graphs pay off where a step is many dependent kernels: the per-operator path
-// (62 kernels per global step, 85-101 per local half) and the sampled local half
-// of the fused path (17 local launches with a sampler after each).  The fused
-// global step and the fused greedy local half are one kernel each, launched
-// directly: a one-node graph measured 14 us per frame slower than the two plain
-// launches (0.432 vs 0.418 ms/frame).
+// (62 kernels per global step, 85-101 per local half).  The fused global step and
+// the fused local half are one kernel each, launched directly: a one-node graph
+// measured 14 us per frame slower than the two plain launches (0.432 vs 0.418
+// ms/frame).
 void Model::build_graphs() {
+    if (fused_layers_) return;
     hipGraph_t g = nullptr;
-    if (!fused_layers_) {
-        hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
-        enqueue_global_step(stream_,
-                            reinterpret_cast<const int *>(reinterpret_cast<uint8_t *>(state_) + kStateRowOff));
-        hip_check(hipStreamEndCapture(stream_, &g), "end capture");
-        hip_check(hipGraphInstantiate(&g_global_, g, nullptr, nullptr, 0), "instantiate global");
-        (void)hipGraphDestroy(g);
-    }
+    hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
+    enqueue_global_step(stream_, reinterpret_cast<const int *>(reinterpret_cast<uint8_t *>(state_) + kStateRowOff));
+    hip_check(hipStreamEndCapture(stream_, &g), "end capture");
+    hip_check(hipGraphInstantiate(&g_global_, g, nullptr, nullptr, 0), "instantiate global");
+    (void)hipGraphDestroy(g);
     for (int fused = 0; fused < 2; ++fused) {
-        if (fused_layers_ && fused) continue;
         hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
         enqueue_frame_local(stream_, false, fused != 0);
         hip_check(hipStreamEndCapture(stream_, &g), "end capture");

@@ -441,7 +441,7 @@ struct LocalArgs {
     const float *x_slot = nullptr;     // lpos 1: the raw input row (dequantised wte[slot])
     const float *qkv_table = nullptr;  // [1 + 15 * 1024][2304]: row 0 for lpos 1, then (lpos, code) rows
     const uint8_t *aemb[kNVq] = {};    // audio embeddings / tied heads
-    int pick = 0;                      // 1: greedy pick of the previous channel here; 0: the sampler wrote state->row
+    int sampled = 0;                   // 1: the call may draw its codes (state->cfg, state->rng), 0: greedy picks only
     int head = 0;                      // 1: position lpos >= 1 also runs the audio head of channel lpos - 1
     float *logits = nullptr;           // [16][1024] head outputs (channel ch at ch * 1024)
     int *counts = nullptr;             // [16][1024] repetition counts (the final pick adds the frame's codes)
@@ -449,7 +449,7 @@ struct LocalArgs {
     float *x_out = nullptr;            // block output (768)
     int gate = 0;                      // 1: after position 0, the W8A8 end gate (wte rows 7, 9); a stop ends the launch
     const uint8_t *wte = nullptr;
-    int final_pick = 0;                // 1: after the last position, the greedy pick of its channel, the
+    int final_pick = 0;                // 1: after the last position, the pick of its channel, the
                                        // frame's code counts, row[0] = slot and frame + 1 (sample_kernel's work)
     int a8 = 0;                        // W8A8 GEMVs (activations quantised per 32-block), else W8A16
     int poll_budget = 0;               // poll rounds a wait may take before it gives up (kPollBudget)
