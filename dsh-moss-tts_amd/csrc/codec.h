@@ -31,6 +31,7 @@ constexpr int kCodecDModel = 256, kCodecHeads = 4, kCodecHeadDim = 64;
 constexpr int kCodecNq = 16, kCodecCb = 1024, kCodecCbDim = 8, kCodecZ = 512;
 constexpr int kCodecStages = 4;
 constexpr int kCodecFinalPatch = 240;
+constexpr int kCodecMaxSplits = 12;  // key splits of an attention launch (its merge holds them all in registers)
 
 // Activation source of a codec GEMM (staged into LDS as fp32, 16 rows at a time).
 enum CodecPro : int {
@@ -64,7 +65,7 @@ struct CodecGemmArgs {
     float *q = nullptr, *kc = nullptr, *vc = nullptr;
     int ring = 0;
     const int *pos0 = nullptr;
-    const float *freq = nullptr;  // [32] RoPE frequencies (host-computed as the reference does)
+    const float2 *rope = nullptr;  // [M][32] (cos, sin) of the rows' positions
 };
 
 struct CodecAttnArgs {
@@ -72,15 +73,19 @@ struct CodecAttnArgs {
     const float *kc = nullptr, *vc = nullptr;  // ring [ring][256]
     int ring = 0, window = 0, M = 0, splits = 1;
     const int *pos0 = nullptr;
-    float *o = nullptr;   // [splits][M][256] unnormalised partial outputs
-    float2 *st = nullptr; // [splits][M][heads] (running max, sum of exponentials)
+    float *o = nullptr;   // [splits][M][256] unnormalised partial outputs; splits == 1: the finished rows
+    float2 *st = nullptr; // [splits][M][heads] (running max, sum of exponentials), splits > 1
 };
 
 struct CodecFrontArgs {
-    const int32_t *codes = nullptr;  // [16][frames]
-    int frames = 0;
+    const int32_t *codes = nullptr;  // row i of the 16 at codes + i * code_stride
+    int code_stride = 0, frames = 0;
     const float *cb[kCodecNq], *cw[kCodecNq], *cbias[kCodecNq];  // [1024][8], [512][8], [512]
     float *z = nullptr;  // [frames][512]
+    const int *pos0 = nullptr;     // [4] the stages' first positions
+    int rows[kCodecStages] = {};   // and row counts of this piece
+    const float *freq = nullptr;   // [32] RoPE frequencies (host-computed as the reference does)
+    float2 *rope[kCodecStages] = {};  // out: [rows][32] (cos, sin)
 };
 
 int codec_gemm_launch(int pro, int epi, const CodecGemmArgs &g, hipStream_t s);
@@ -91,7 +96,18 @@ int codec_advance_launch(int *pos0, const int *rows, hipStream_t s);  // pos0[i]
 // One stream's decoder state: per stage the next position and per layer the K/V rings.
 struct CodecState {
     int *pos0 = nullptr;  // device [4]
+    int ring[kCodecStages] = {};
     std::vector<float *> k, v;  // per layer (all stages, in order), [ring_s][256] each
+};
+
+// The activations of one piece of at most `cap` frames.
+struct CodecWork {
+    int cap = 0;
+    int32_t *codes = nullptr;
+    size_t codes_cap = 0;
+    float *z = nullptr, *xa = nullptr, *xb = nullptr, *y = nullptr, *qb = nullptr, *h = nullptr;
+    float *ao = nullptr, *out = nullptr;
+    float2 *ast = nullptr, *rope = nullptr;
 };
 
 class Codec {
@@ -121,14 +137,18 @@ private:
     struct StageW {
         const void *in, *out;
         int in_f32, out_f32;
-        int cin, cout, patch, window, ring, layer0, nlayers;
+        int cin, cout, patch, window, layer0, nlayers;
     };
-    void alloc_state(CodecState &st);
+    void alloc_state(CodecState &st, int frames);
     void free_state(CodecState &st);
     void clear_state(CodecState &st);
-    // launches of one piece of <= fmax_ frames (codes already in codes_dev_), samples to out_dev_;
-    // stage_ev (5 events, [0] recorded by the caller) marks each stage's end
-    void enqueue(CodecState &st, int frames, hipEvent_t *stage_ev);
+    void alloc_work(CodecWork &w, int frames);
+    void free_work(CodecWork &w);
+    void ensure_whole(int piece, int frames);
+    // launches of one piece of <= w.cap frames (codes on the device, `stride` apart per
+    // quantizer), samples to w.out; stage_ev (5 events, [0] recorded by the caller) marks each
+    // stage's end
+    void enqueue(CodecState &st, CodecWork &w, const int32_t *codes, int stride, int frames, hipEvent_t *stage_ev);
     int splits_for(int stage, int rows) const;
     void check_codes(const int32_t *codes, int frames) const;
     void run_piece(CodecState &st, const int32_t *codes, int frames, float *out, bool graph);
@@ -144,22 +164,16 @@ private:
     StageW stages_[kCodecStages];
     std::vector<LayerW> layers_;
     float *freq_ = nullptr;  // device [32]
-    // activations
-    int32_t *codes_dev_ = nullptr;
-    float *z_ = nullptr, *xa_ = nullptr, *xb_ = nullptr, *y_ = nullptr, *qb_ = nullptr, *h_ = nullptr;
-    float *ao_ = nullptr;
-    float2 *ast_ = nullptr;
-    float *out_dev_ = nullptr;
+    int c0_ = 0;             // q.out rows: the first stage's input width before its patch
+    CodecWork work_, whole_work_;
     int32_t *codes_host_ = nullptr;  // pinned staging
     float *out_host_ = nullptr;
-    size_t out_host_cap_ = 0;
+    float *whole_host_[2] = {};      // decode(): the samples of two pieces, pinned
     CodecState stream_state_, whole_state_;
-    bool whole_alloc_ = false;
     std::map<int, hipGraphExec_t> graphs_;  // per piece size (frames), stream state
-    hipEvent_t ev_[kCodecStages + 1] = {};
+    hipEvent_t ev_[2][kCodecStages + 1] = {}, done_[2] = {};
     double last_ms_ = 0.0, stage_ms_[kCodecStages] = {0, 0, 0, 0};
     std::string info_;
-    int max_splits_ = 1;
     bool eager_ = false;
 };
 

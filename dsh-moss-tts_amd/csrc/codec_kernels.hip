@@ -56,6 +56,35 @@ struct W8 {
     }
 };
 
+// RoPE of a QKV column: pairs (2i, 2i+1), angle = float(pos) * freq in fp32 (audio_rope,
+// audio_layer.cpp:30-44), cos and sin from the piece's table; q to its buffer, k and v to the
+// ring slot of the row's position.
+__device__ __forceinline__ void qkv_store(const CodecGemmArgs &g, int m, int nn, float v, float partner) {
+    const int region = nn / kCodecDModel, c = nn - region * kCodecDModel;
+    float out = v;
+    if (region < 2) {
+        const float2 cs = g.rope[(size_t)m * (kCodecHeadDim / 2) + ((c & (kCodecHeadDim - 1)) >> 1)];
+        out = (c & 1) ? partner * cs.y + v * cs.x : v * cs.x - partner * cs.y;
+    }
+    float *dst = region == 0 ? g.q : (region == 1 ? g.kc : g.vc);
+    const size_t row = region == 0 ? (size_t)m : (size_t)((*g.pos0 + m) % g.ring);
+    dst[row * kCodecDModel + c] = out;
+}
+
+template <int EPI>
+__device__ __forceinline__ void epi_store(const CodecGemmArgs &g, int m, int nn, float v) {
+    if constexpr (EPI == CEPI_STORE) {
+        const int p = g.patch;
+        g.y[((size_t)m * p + nn % p) * g.ldy + nn / p] = g.bias ? v + g.bias[nn] : v;
+    } else if constexpr (EPI == CEPI_GELU) {
+        // audio_gelu (audio_layer.cpp:46)
+        g.y[(size_t)m * g.ldy + nn] = 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
+    } else {
+        float *y = g.y + (size_t)m * g.ldy + nn;
+        *y = *y + g.ls[nn] * v;
+    }
+}
+
 // Y[m][n] = sum_k A[m][k] W[n][k] over a 16-row x 16-column tile.  The contraction is
 // cut into chunks of 32 columns; wave w takes chunks [w nch/4, (w+1) nch/4) of every
 // round of 1024 columns and reads its A and W straight from global memory (each lane
@@ -75,19 +104,25 @@ __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) 
     const bool avalid = am < g.M;
     const int n = n0 + col;          // W row this lane feeds (N % 16 == 0: always valid)
 
-    // CPRO_MERGE: this lane's (row am, head = wave) split weights e^(m_s - M) / sum_s e^(m_s - M) l_s
-    float mx = 0.f, inv_den = 0.f;
+    // CPRO_MERGE: this lane's (row am, head = wave) split weights e^(m_s - M) / sum_s e^(m_s - M) l_s.
+    // Every split's statistics are loaded before any is used (a loop over the splits waited for
+    // each in turn: 10.7 us for the proj launch of an 8-frame chunk)
+    float fs[PRO == CPRO_MERGE ? kCodecMaxSplits : 1], inv_den = 0.f;
     if constexpr (PRO == CPRO_MERGE) {
-        if (avalid) {
-            mx = -INFINITY;
-            for (int s = 0; s < g.splits; ++s) mx = fmaxf(mx, g.st[((size_t)s * g.M + am) * kCodecHeads + wave].x);
-            float den = 0.f;
-            for (int s = 0; s < g.splits; ++s) {
-                const float2 st = g.st[((size_t)s * g.M + am) * kCodecHeads + wave];
-                den += exp_f(st.x - mx) * st.y;
-            }
-            inv_den = 1.0f / den;
+        float2 st[kCodecMaxSplits];
+        const float2 *sp = g.st + (size_t)(avalid ? am : 0) * kCodecHeads + wave;
+#pragma unroll
+        for (int s = 0; s < kCodecMaxSplits; ++s)
+            st[s] = s < g.splits ? sp[(size_t)s * g.M * kCodecHeads] : make_float2(-INFINITY, 0.f);
+        float mx = -INFINITY, den = 0.f;
+#pragma unroll
+        for (int s = 0; s < kCodecMaxSplits; ++s) mx = fmaxf(mx, st[s].x);
+#pragma unroll
+        for (int s = 0; s < kCodecMaxSplits; ++s) {
+            fs[s] = s < g.splits ? exp_f(st[s].x - mx) : 0.f;
+            den += fs[s] * st[s].y;
         }
+        inv_den = 1.0f / den;
     }
 
     floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
@@ -102,23 +137,29 @@ __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) 
             if (c0 + c < c1) {
                 wr[c].load(g.w, (size_t)n * g.K + kk);
                 if constexpr (PRO == CPRO_MERGE) {
-                    av[c][0] = av[c][1] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (avalid) {
-                        for (int s = 0; s < g.splits; ++s) {
-                            const float2 st = g.st[((size_t)s * g.M + am) * kCodecHeads + wave];
-                            const float f = exp_f(st.x - mx);
-                            const float4 *o = reinterpret_cast<const float4 *>(g.o + ((size_t)s * g.M + am) * kCodecDModel + kk);
-                            const float4 o0 = o[0], o1 = o[1];
-                            av[c][0].x += f * o0.x;
-                            av[c][0].y += f * o0.y;
-                            av[c][0].z += f * o0.z;
-                            av[c][0].w += f * o0.w;
-                            av[c][1].x += f * o1.x;
-                            av[c][1].y += f * o1.y;
-                            av[c][1].z += f * o1.z;
-                            av[c][1].w += f * o1.w;
+                    const float *op = g.o + (size_t)(avalid ? am : 0) * kCodecDModel + kk;
+                    float4 o[kCodecMaxSplits][2];
+#pragma unroll
+                    for (int s = 0; s < kCodecMaxSplits; ++s)
+                        if (s < g.splits) {  // (uniform)
+                            const float4 *os = reinterpret_cast<const float4 *>(op + (size_t)s * g.M * kCodecDModel);
+                            o[s][0] = os[0];
+                            o[s][1] = os[1];
                         }
-                    }
+                    av[c][0] = av[c][1] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                    for (int s = 0; s < kCodecMaxSplits; ++s)
+                        if (s < g.splits && avalid) {
+                            const float f = fs[s];
+                            av[c][0].x += f * o[s][0].x;
+                            av[c][0].y += f * o[s][0].y;
+                            av[c][0].z += f * o[s][0].z;
+                            av[c][0].w += f * o[s][0].w;
+                            av[c][1].x += f * o[s][1].x;
+                            av[c][1].y += f * o[s][1].y;
+                            av[c][1].z += f * o[s][1].z;
+                            av[c][1].w += f * o[s][1].w;
+                        }
                 } else {
                     const float4 *src = reinterpret_cast<const float4 *>(g.a + (size_t)(avalid ? am : 0) * g.lda + kk);
                     av[c][0] = avalid ? src[0] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -186,31 +227,171 @@ __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) 
     if (m >= g.M) return;
 
     if constexpr (EPI == CEPI_QKV) {
-        const int region = nn / kCodecDModel, c = nn - region * kCodecDModel;
-        const int pos = *g.pos0 + m;
-        float out = v;
-        if (region < 2) {
-            // audio_rope (audio_layer.cpp:30-44): pairs (2i, 2i+1), angle = float(pos) * freq in fp32
-            const int tp = t ^ 1;
-            const float partner = (red[0][tp] + red[1][tp]) + (red[2][tp] + red[3][tp]);
-            const float ang = (float)pos * g.freq[(c & (kCodecHeadDim - 1)) >> 1];
-            float sn, cs;
-            sincosf(ang, &sn, &cs);
-            out = (c & 1) ? partner * sn + v * cs : v * cs - partner * sn;
-        }
-        float *dst = region == 0 ? g.q : (region == 1 ? g.kc : g.vc);
-        const size_t row = region == 0 ? (size_t)m : (size_t)(pos % g.ring);
-        dst[row * kCodecDModel + c] = out;
-    } else if constexpr (EPI == CEPI_STORE) {
-        const int p = g.patch;
-        g.y[((size_t)m * p + nn % p) * g.ldy + nn / p] = g.bias ? v + g.bias[nn] : v;
-    } else if constexpr (EPI == CEPI_GELU) {
-        // audio_gelu (audio_layer.cpp:46)
-        g.y[(size_t)m * g.ldy + nn] = 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
+        const int tp = t ^ 1;
+        qkv_store(g, m, nn, v, (red[0][tp] + red[1][tp]) + (red[2][tp] + red[3][tp]));
     } else {
-        float *y = g.y + (size_t)m * g.ldy + nn;
-        *y = *y + g.ls[nn] * v;
+        epi_store<EPI>(g, m, nn, v);
     }
+}
+
+// The same product for pieces with many rows: a workgroup takes 32 MT rows x 32 NT columns,
+// its 4 waves 2 x 2 of 16 MT x 16 NT, each over the whole contraction.  What bounds it is the
+// fp32 matrix rate (64 flop per SIMD and cycle), so operands come straight from global memory
+// -- per 32 columns a wave loads 2 MT + NT vectors for 8 MT NT MFMAs of 32 cycles -- with the next
+// chunk in flight.  CPRO_LN (K = 256): the rows are read once, 8 / MT threads a row, normalised
+// in registers and kept in LDS (rows of 260 floats: the 16 rows of a 16-byte read fall into
+// different banks).  Consecutive workgroups go to different XCDs, so the tiles are numbered
+// such that all column tiles of a row tile run on one XCD and its L2 holds their rows.
+// (An utterance of 203 frames, with decode()'s long pieces: 6.66 ms in 32-frame pieces of 16 x 16
+// tiles, 3.30 ms.)
+template <int PRO, int EPI, int WF32, int MT, int NT>
+__global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, int ntiles, int mtiles) {
+    constexpr int kLdA = kCodecDModel + 4;
+    __shared__ float as[PRO == CPRO_LN ? 32 * MT : 1][kLdA];
+    const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
+    const int mt0 = (slot / ntiles) * 8 + xcd;
+    if (mt0 >= mtiles) return;
+    const int m0 = mt0 * 32 * MT, n0 = (slot % ntiles) * 32 * NT;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, col = lane & 15, grp = lane >> 4;
+    const int wm = (wave >> 1) * 16 * MT, wn = n0 + (wave & 1) * 16 * NT;
+
+    size_t woff[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) woff[j] = (size_t)min(wn + 16 * j + col, g.N - 1) * g.K + 8 * grp;
+    const float *arow[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) arow[i] = g.a + (size_t)min(m0 + wm + 16 * i + col, g.M - 1) * g.lda + 8 * grp;
+
+    W8<WF32> wr[2][NT];
+    float4 av[2][MT][2];
+    auto load = [&](int s, int kk) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) wr[s][j].load(g.w, woff[j] + kk);
+        if constexpr (PRO != CPRO_LN)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const float4 *p = reinterpret_cast<const float4 *>(arow[i] + kk);
+                av[s][i][0] = p[0];
+                av[s][i][1] = p[1];
+            }
+    };
+    load(0, 0);
+    if constexpr (PRO == CPRO_LN) {
+        // audio_layernorm (audio_layer.cpp:17-28): two-pass mean / variance over 256, eps 1e-5
+        constexpr int TPR = 8 / MT, V = kCodecDModel / 4 / TPR;  // threads and float4s per row
+        const int r = t / TPR, q = t % TPR;
+        const float4 *src = reinterpret_cast<const float4 *>(g.a + (size_t)min(m0 + r, g.M - 1) * g.lda) + q;
+        float4 x[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) x[i] = src[TPR * i];
+        auto row_sum = [&](float v) {
+            v += xshfl<1>(v);
+            v += xshfl<2>(v);
+            if constexpr (TPR == 8) v += xshfl<4>(v);
+            return v;
+        };
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < V; ++i) sum += (x[i].x + x[i].y) + (x[i].z + x[i].w);
+        const float mean = row_sum(sum) / 256.0f;
+        float sq = 0.f;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            x[i].x -= mean;
+            x[i].y -= mean;
+            x[i].z -= mean;
+            x[i].w -= mean;
+            sq += (x[i].x * x[i].x + x[i].y * x[i].y) + (x[i].z * x[i].z + x[i].w * x[i].w);
+        }
+        const float inv = 1.0f / sqrtf(row_sum(sq) / 256.0f + 1e-5f);
+        const float4 *lw = reinterpret_cast<const float4 *>(g.ln_w) + q, *lb = reinterpret_cast<const float4 *>(g.ln_b) + q;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            const float4 w = lw[TPR * i], b = lb[TPR * i];
+            *reinterpret_cast<float4 *>(&as[r][4 * (q + TPR * i)]) =
+                make_float4(x[i].x * inv * w.x + b.x, x[i].y * inv * w.y + b.y, x[i].z * inv * w.z + b.z,
+                            x[i].w * inv * w.w + b.w);
+        }
+        lds_barrier();
+    }
+
+    // sums of 64 columns at a time, then those (one chain over K = 1024 measured twice the error
+    // of the sums split over waves, 7e-7 against 4e-7 after all layers)
+    floatx4 acc[MT][NT], tot[MT][NT];
+    auto clear = [](floatx4 (&v)[MT][NT]) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) v[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    };
+    auto flush = [&] {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) tot[i][j] += acc[i][j];
+        clear(acc);
+    };
+    clear(acc);
+    clear(tot);
+    auto step = [&](int s, int kk) {
+        float a[MT][8];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            float4 x0, x1;
+            if constexpr (PRO == CPRO_LN) {
+                const float4 *p = reinterpret_cast<const float4 *>(&as[wm + 16 * i + col][kk + 8 * grp]);
+                x0 = p[0];
+                x1 = p[1];
+            } else {
+                x0 = av[s][i][0];
+                x1 = av[s][i][1];
+            }
+            a[i][0] = x0.x;
+            a[i][1] = x0.y;
+            a[i][2] = x0.z;
+            a[i][3] = x0.w;
+            a[i][4] = x1.x;
+            a[i][5] = x1.y;
+            a[i][6] = x1.z;
+            a[i][7] = x1.w;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = mfma4(a[i][k], wr[s][j].get(k), acc[i][j]);
+    };
+    int kk = 0;
+    for (; kk + 64 <= g.K; kk += 64) {
+        load(1, kk + 32);
+        step(0, kk);
+        if (kk + 64 < g.K) load(0, kk + 64);
+        step(1, kk + 32);
+        flush();
+    }
+    if (kk < g.K) {  // K an odd number of chunks
+        step(0, kk);
+        flush();
+    }
+
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + wm + 16 * i + 4 * grp + e;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const int nn = wn + 16 * j + col;
+                const float v = tot[i][j][e];
+                if constexpr (EPI == CEPI_QKV) {
+                    const float partner = xshfl<1>(v);
+                    if (m < g.M && nn < g.N) qkv_store(g, m, nn, v, partner);
+                } else {
+                    if (m < g.M && nn < g.N) epi_store<EPI>(g, m, nn, v);
+                }
+            }
+        }
 }
 
 // Windowed causal attention of 16 query rows x one head over the ring's keys
@@ -353,29 +534,63 @@ __global__ __launch_bounds__(256) void codec_attn_kernel(const CodecAttnArgs a) 
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[e] += f * red[w][(4 * d4 + e) * 16 + q];
     }
+    if (a.splits == 1) {
+        const float inv = 1.0f / l;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] *= inv;
+    }
     const size_t row = (size_t)split * a.M + m;
     *reinterpret_cast<float4 *>(a.o + row * kCodecDModel + hoff + 4 * d4) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    if (d4 == 0) a.st[row * kCodecHeads + h] = make_float2(mx, l);
+    if (d4 == 0 && a.splits > 1) a.st[row * kCodecHeads + h] = make_float2(mx, l);
 }
 
-// z[t][r] = sum_i (b_i[r] + sum_k W_i[r][k] cb_i[code_it][k])   (decoder.cpp:224-240)
+// Workgroup t < frames: z[t][r] = sum_i (b_i[r] + sum_k W_i[r][k] cb_i[code_it][k]), i in order
+// (decoder.cpp:224-240); the 16 quantizers' loads are all in flight together (one after the
+// other: 9.1 us).  The workgroups after those: cos and sin of every stage's positions, which
+// each layer's q and k then read (sincosf per element of every QKV launch before).
 __global__ __launch_bounds__(512) void codec_front_kernel(const CodecFrontArgs a) {
+    if ((int)blockIdx.x >= a.frames) {
+        int e = ((int)blockIdx.x - a.frames) * 512 + threadIdx.x;  // entry: stage, row, frequency
+        const int f = e & 31;
+        e >>= 5;
+#pragma unroll
+        for (int s = 0; s < kCodecStages; ++s) {
+            if (e < a.rows[s]) {
+                float sn, cs;
+                sincosf((float)(a.pos0[s] + e) * a.freq[f], &sn, &cs);
+                a.rope[s][(size_t)e * 32 + f] = make_float2(cs, sn);
+                return;
+            }
+            e -= a.rows[s];
+        }
+        return;
+    }
     const int t = blockIdx.x, r = threadIdx.x;
-    float z = 0.f;
+    float4 e0[kCodecNq], e1[kCodecNq], w0[kCodecNq], w1[kCodecNq];
+    float b[kCodecNq];
+#pragma unroll
     for (int i = 0; i < kCodecNq; ++i) {
-        const int code = a.codes[i * a.frames + t];
+        const int code = a.codes[(size_t)i * a.code_stride + t];
         const float4 *e = reinterpret_cast<const float4 *>(a.cb[i] + (size_t)code * kCodecCbDim);
         const float4 *w = reinterpret_cast<const float4 *>(a.cw[i] + (size_t)r * kCodecCbDim);
-        const float4 e0 = e[0], e1 = e[1], w0 = w[0], w1 = w[1];
-        float acc = a.cbias[i][r];
-        acc += w0.x * e0.x;
-        acc += w0.y * e0.y;
-        acc += w0.z * e0.z;
-        acc += w0.w * e0.w;
-        acc += w1.x * e1.x;
-        acc += w1.y * e1.y;
-        acc += w1.z * e1.z;
-        acc += w1.w * e1.w;
+        e0[i] = e[0];
+        e1[i] = e[1];
+        w0[i] = w[0];
+        w1[i] = w[1];
+        b[i] = a.cbias[i][r];
+    }
+    float z = 0.f;
+#pragma unroll
+    for (int i = 0; i < kCodecNq; ++i) {
+        float acc = b[i];
+        acc += w0[i].x * e0[i].x;
+        acc += w0[i].y * e0[i].y;
+        acc += w0[i].z * e0[i].z;
+        acc += w0[i].w * e0[i].w;
+        acc += w1[i].x * e1[i].x;
+        acc += w1[i].y * e1[i].y;
+        acc += w1[i].z * e1[i].z;
+        acc += w1[i].w * e1[i].w;
         z += acc;
     }
     a.z[(size_t)t * kCodecZ + r] = z;
@@ -389,9 +604,33 @@ __global__ void codec_advance_kernel(int *pos0, Rows4 rows) {
     if (threadIdx.x < kCodecStages) pos0[threadIdx.x] += rows.r[threadIdx.x];
 }
 
+// Tiles of 64 x 64, or else 32 x 32, from this many of them on.
+constexpr long kTile64Min = 192, kTile32Min = 256;
+
+template <int PRO, int EPI, int MT, int NT>
+void launch_tile(const CodecGemmArgs &g, hipStream_t s) {
+    const int mt = (g.M + 32 * MT - 1) / (32 * MT), nt = (g.N + 32 * NT - 1) / (32 * NT);
+    const dim3 grid(8 * nt * ((mt + 7) / 8));
+    if (g.w_f32)
+        hipLaunchKernelGGL((codec_tile_kernel<PRO, EPI, 1, MT, NT>), grid, dim3(256), 0, s, g, nt, mt);
+    else
+        hipLaunchKernelGGL((codec_tile_kernel<PRO, EPI, 0, MT, NT>), grid, dim3(256), 0, s, g, nt, mt);
+}
+
 template <int PRO, int EPI>
 int launch_w(const CodecGemmArgs &g, hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
+    if constexpr (PRO != CPRO_MERGE) {
+        const long tiles64 = (long)((g.M + 63) / 64) * ((g.N + 63) / 64), tiles32 = (long)((g.M + 31) / 32) * ((g.N + 31) / 32);
+        if (tiles64 >= kTile64Min) {
+            launch_tile<PRO, EPI, 2, 2>(g, s);
+            return hipGetLastError() == hipSuccess ? 0 : MOSS_HIP_EDEVICE;
+        }
+        if (tiles32 >= kTile32Min) {
+            launch_tile<PRO, EPI, 1, 1>(g, s);
+            return hipGetLastError() == hipSuccess ? 0 : MOSS_HIP_EDEVICE;
+        }
+    }
     const dim3 grid(g.N / 16, (g.M + 15) / 16);
     if (g.w_f32)
         hipLaunchKernelGGL((codec_gemm_kernel<PRO, EPI, 1>), grid, dim3(256), 0, s, g);
@@ -407,8 +646,8 @@ int codec_gemm_launch(int pro, int epi, const CodecGemmArgs &g, hipStream_t s) {
         return MOSS_HIP_EINVAL;
     if ((pro == CPRO_LN || pro == CPRO_MERGE) && g.K != kCodecDModel) return MOSS_HIP_EINVAL;
     if (pro == CPRO_ROWS && (g.lda % 4 || g.lda < g.K)) return MOSS_HIP_EINVAL;
-    if (pro == CPRO_MERGE && (!g.o || !g.st || g.splits < 1)) return MOSS_HIP_EINVAL;
-    if (epi == CEPI_QKV && (g.N != 3 * kCodecDModel || !g.q || !g.kc || !g.vc || g.ring <= 0 || !g.pos0 || !g.freq))
+    if (pro == CPRO_MERGE && (!g.o || !g.st || g.splits < 1 || g.splits > kCodecMaxSplits)) return MOSS_HIP_EINVAL;
+    if (epi == CEPI_QKV && (g.N != 3 * kCodecDModel || !g.q || !g.kc || !g.vc || g.ring <= 0 || !g.pos0 || !g.rope))
         return MOSS_HIP_EINVAL;
     if (epi == CEPI_STORE && (g.patch < 1 || g.N % g.patch)) return MOSS_HIP_EINVAL;
     if (epi == CEPI_RESID && !g.ls) return MOSS_HIP_EINVAL;
@@ -433,8 +672,14 @@ int codec_attn_launch(const CodecAttnArgs &a, hipStream_t s) {
 
 int codec_front_launch(const CodecFrontArgs &a, hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
-    if (a.frames <= 0 || !a.codes || !a.z) return MOSS_HIP_EINVAL;
-    hipLaunchKernelGGL(codec_front_kernel, dim3(a.frames), dim3(kCodecZ), 0, s, a);
+    if (a.frames <= 0 || !a.codes || !a.z || a.code_stride < a.frames || !a.pos0 || !a.freq) return MOSS_HIP_EINVAL;
+    long rows = 0;
+    for (int i = 0; i < kCodecStages; ++i) {
+        if (a.rows[i] <= 0 || !a.rope[i]) return MOSS_HIP_EINVAL;
+        rows += a.rows[i];
+    }
+    const dim3 grid(a.frames + (unsigned)((rows * 32 + 511) / 512));
+    hipLaunchKernelGGL(codec_front_kernel, grid, dim3(kCodecZ), 0, s, a);
     return hipGetLastError() == hipSuccess ? 0 : MOSS_HIP_EDEVICE;
 }
 

@@ -17,6 +17,8 @@ constexpr int kLayerCounts[kCodecStages] = {4, 2, 2, 4};    // decoder.cpp:44
 constexpr int kContexts[kCodecStages] = {500, 800, 1200, 1600};  // decoder.cpp:21
 constexpr int kDtF16 = 0, kDtF32 = 3;  // DType (csrc/include/moss/common.h:26)
 constexpr int kMaxPieceFrames = 1024;
+// decode() runs an utterance in equal pieces of at most this many frames
+constexpr int kWholePiece = 104;
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
@@ -111,7 +113,6 @@ Codec::Codec(const void *blob, size_t bytes, const moss_hip_codec_options &opt) 
         S.window = opt.contexts[s] > 0 ? opt.contexts[s] : kContexts[s];
         S.layer0 = (int)layers_.size();
         S.nlayers = kLayerCounts[s];
-        S.ring = S.window + stage_rows(fmax_, s);
         for (int n = 0; n < S.nlayers; ++n) {
             const std::string lp = p + "l" + std::to_string(n) + ".";
             LayerW L{};
@@ -179,33 +180,14 @@ Codec::Codec(const void *blob, size_t bytes, const moss_hip_codec_options &opt) 
     hip_check(hipMalloc(&freq_, sizeof(freq)), "hipMalloc(freq)");
     hip_check(hipMemcpy(freq_, freq, sizeof(freq), hipMemcpyHostToDevice), "upload freq");
 
-    // activations, sized for pieces of fmax_ frames
-    size_t xmax = (size_t)fmax_ * c0;  // q.out output = stage 0 input
-    for (int s = 0; s + 1 < kCodecStages; ++s) xmax = std::max(xmax, (size_t)stage_rows(fmax_, s) * stages_[s].cout);
-    const size_t rmax = (size_t)stage_rows(fmax_, kCodecStages - 1);
-    size_t part_rows = 0;
-    for (int f = 1; f <= fmax_; ++f)
-        for (int s = 0; s < kCodecStages; ++s) {
-            const int r = stage_rows(f, s);
-            max_splits_ = std::max(max_splits_, splits_for(s, r));
-            part_rows = std::max(part_rows, (size_t)splits_for(s, r) * r);
-        }
-    auto fmalloc = [&](float **p, size_t n) { hip_check(hipMalloc(p, std::max<size_t>(n, 64) * 4), "hipMalloc(codec act)"); };
-    hip_check(hipMalloc(&codes_dev_, sizeof(int32_t) * kCodecNq * fmax_), "hipMalloc(codes)");
-    fmalloc(&z_, (size_t)fmax_ * kCodecZ);
-    fmalloc(&xa_, xmax);
-    fmalloc(&xb_, xmax);
-    fmalloc(&y_, rmax * kCodecDModel);
-    fmalloc(&qb_, rmax * kCodecDModel);
-    fmalloc(&h_, rmax * ffn_max_);
-    fmalloc(&ao_, part_rows * kCodecDModel);
-    hip_check(hipMalloc(&ast_, sizeof(float2) * part_rows * kCodecHeads), "hipMalloc(attn stats)");
-    fmalloc(&out_dev_, (size_t)fmax_ * spf_);
+    c0_ = c0;
+    alloc_work(work_, fmax_);
     hip_check(hipHostMalloc(&codes_host_, sizeof(int32_t) * kCodecNq * fmax_), "hipHostMalloc(codes)");
-    out_host_cap_ = (size_t)fmax_ * spf_;
-    hip_check(hipHostMalloc(&out_host_, sizeof(float) * out_host_cap_), "hipHostMalloc(samples)");
-    for (auto &e : ev_) hip_check(hipEventCreate(&e), "hipEventCreate");
-    alloc_state(stream_state_);
+    hip_check(hipHostMalloc(&out_host_, sizeof(float) * (size_t)fmax_ * spf_), "hipHostMalloc(samples)");
+    for (auto &set : ev_)
+        for (auto &e : set) hip_check(hipEventCreate(&e), "hipEventCreate");
+    for (auto &e : done_) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+    alloc_state(stream_state_, fmax_);
     clear_state(stream_state_);
     hip_check(hipStreamSynchronize(stream_), "codec init");
 
@@ -221,14 +203,20 @@ Codec::~Codec() {
     if (stream_) (void)hipStreamSynchronize(stream_);
     for (auto &kv : graphs_) (void)hipGraphExecDestroy(kv.second);
     free_state(stream_state_);
-    if (whole_alloc_) free_state(whole_state_);
-    for (auto &e : ev_)
+    free_state(whole_state_);
+    free_work(work_);
+    free_work(whole_work_);
+    for (auto &set : ev_)
+        for (auto &e : set)
+            if (e) (void)hipEventDestroy(e);
+    for (auto &e : done_)
         if (e) (void)hipEventDestroy(e);
-    void *dev[] = {wdev_, freq_, codes_dev_, z_, xa_, xb_, y_, qb_, h_, ao_, ast_, out_dev_};
-    for (void *p : dev)
-        if (p) (void)hipFree(p);
+    if (wdev_) (void)hipFree(wdev_);
+    if (freq_) (void)hipFree(freq_);
     if (codes_host_) (void)hipHostFree(codes_host_);
     if (out_host_) (void)hipHostFree(out_host_);
+    for (float *p : whole_host_)
+        if (p) (void)hipHostFree(p);
     if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -240,15 +228,79 @@ int Codec::splits_for(int stage, int rows) const {
     const int tiles = (rows + 15) / 16;
     const int blocks = (stages_[stage].window + 15 + 15) / 16;
     const int want = (512 + tiles * kCodecHeads - 1) / (tiles * kCodecHeads);
-    return std::max(1, std::min(want, blocks / 8));
+    return std::max(1, std::min(std::min(want, blocks / 8), kCodecMaxSplits));
 }
 
-void Codec::alloc_state(CodecState &st) {
+// Buffers for pieces of up to `frames` frames.
+void Codec::alloc_work(CodecWork &w, int frames) {
+    size_t xmax = (size_t)frames * c0_;  // q.out output = stage 0 input
+    for (int s = 0; s + 1 < kCodecStages; ++s) xmax = std::max(xmax, (size_t)stage_rows(frames, s) * stages_[s].cout);
+    const size_t rmax = (size_t)stage_rows(frames, kCodecStages - 1);
+    size_t part_rows = 0, rope_rows = 0;
+    for (int f = 1; f <= frames; ++f)
+        for (int s = 0; s < kCodecStages; ++s) {
+            const int r = stage_rows(f, s);
+            part_rows = std::max(part_rows, (size_t)splits_for(s, r) * r);
+        }
+    for (int s = 0; s < kCodecStages; ++s) rope_rows += stage_rows(frames, s);
+    auto fmalloc = [&](float **p, size_t n) { hip_check(hipMalloc(p, std::max<size_t>(n, 64) * 4), "hipMalloc(codec act)"); };
+    w.codes_cap = (size_t)kCodecNq * frames;
+    hip_check(hipMalloc(&w.codes, sizeof(int32_t) * w.codes_cap), "hipMalloc(codes)");
+    fmalloc(&w.z, (size_t)frames * kCodecZ);
+    fmalloc(&w.xa, xmax);
+    fmalloc(&w.xb, xmax);
+    fmalloc(&w.y, rmax * kCodecDModel);
+    fmalloc(&w.qb, rmax * kCodecDModel);
+    fmalloc(&w.h, rmax * ffn_max_);
+    fmalloc(&w.ao, part_rows * kCodecDModel);
+    hip_check(hipMalloc(&w.ast, sizeof(float2) * part_rows * kCodecHeads), "hipMalloc(attn stats)");
+    hip_check(hipMalloc(&w.rope, sizeof(float2) * rope_rows * (kCodecHeadDim / 2)), "hipMalloc(rope)");
+    fmalloc(&w.out, (size_t)frames * spf_);
+    w.cap = frames;
+}
+
+void Codec::free_work(CodecWork &w) {
+    void *dev[] = {w.codes, w.z, w.xa, w.xb, w.y, w.qb, w.h, w.ao, w.ast, w.rope, w.out};
+    for (void *p : dev)
+        if (p) (void)hipFree(p);
+    w = CodecWork{};
+}
+
+// decode()'s own state and buffers, for pieces of `piece` frames of `frames`; they grow to the
+// largest piece asked for (at most kWholePiece frames) and are kept.
+void Codec::ensure_whole(int piece, int frames) {
+    if (piece > whole_work_.cap) {
+        hip_check(hipStreamSynchronize(stream_), "codec decode");
+        free_state(whole_state_);
+        free_work(whole_work_);
+        for (float *&p : whole_host_) {
+            if (p) (void)hipHostFree(p);
+            p = nullptr;
+        }
+        const int cap = std::min((piece + 31) / 32 * 32, kWholePiece);
+        alloc_state(whole_state_, cap);
+        for (float *&p : whole_host_)
+            hip_check(hipHostMalloc(&p, sizeof(float) * (size_t)cap * spf_), "hipHostMalloc(samples)");
+        alloc_work(whole_work_, cap);
+    }
+    const size_t n = (size_t)kCodecNq * frames;
+    if (n > whole_work_.codes_cap) {
+        if (whole_work_.codes) hip_check(hipFree(whole_work_.codes), "free codes");
+        whole_work_.codes = nullptr;
+        whole_work_.codes_cap = 0;
+        hip_check(hipMalloc(&whole_work_.codes, sizeof(int32_t) * n), "hipMalloc(codes)");
+        whole_work_.codes_cap = n;
+    }
+}
+
+// Rings for pieces of up to `frames` frames.
+void Codec::alloc_state(CodecState &st, int frames) {
     hip_check(hipMalloc(&st.pos0, sizeof(int) * kCodecStages), "hipMalloc(codec pos)");
-    for (int s = 0; s < kCodecStages; ++s)
+    for (int s = 0; s < kCodecStages; ++s) {
+        st.ring[s] = stages_[s].window + stage_rows(frames, s);
         for (int n = 0; n < stages_[s].nlayers; ++n) {
             float *k = nullptr, *v = nullptr;
-            const size_t nb = sizeof(float) * stages_[s].ring * kCodecDModel;
+            const size_t nb = sizeof(float) * st.ring[s] * kCodecDModel;
             hip_check(hipMalloc(&k, nb), "hipMalloc(codec ring)");
             hip_check(hipMalloc(&v, nb), "hipMalloc(codec ring)");
             // zero once: a ring slot is only read after this stream wrote it, but keep it finite
@@ -257,6 +309,7 @@ void Codec::alloc_state(CodecState &st) {
             st.k.push_back(k);
             st.v.push_back(v);
         }
+    }
 }
 
 void Codec::free_state(CodecState &st) {
@@ -289,22 +342,31 @@ static void ok(int rc, const char *what) {
 }
 
 // The launches of one piece: front, q.out (+ patch 4), four stages, position advance.
-void Codec::enqueue(CodecState &st, int frames, hipEvent_t *stage_ev) {
+void Codec::enqueue(CodecState &st, CodecWork &w, const int32_t *codes, int stride, int frames, hipEvent_t *stage_ev) {
     hipStream_t s = stream_;
     CodecFrontArgs fa;
-    fa.codes = codes_dev_;
+    fa.codes = codes;
+    fa.code_stride = stride;
     fa.frames = frames;
+    fa.pos0 = st.pos0;
+    fa.freq = freq_;
+    float2 *rope = w.rope;
+    for (int si = 0; si < kCodecStages; ++si) {
+        fa.rows[si] = stage_rows(frames, si);
+        fa.rope[si] = rope;
+        rope += (size_t)fa.rows[si] * (kCodecHeadDim / 2);
+    }
     for (int i = 0; i < kCodecNq; ++i) {
         fa.cb[i] = front_cb_[i];
         fa.cw[i] = front_w_[i];
         fa.cbias[i] = front_b_[i];
     }
-    fa.z = z_;
+    fa.z = w.z;
     ok(codec_front_launch(fa, s), "front");
-    float *xin = xa_, *xother = xb_;
+    float *xin = w.xa, *xother = w.xb;
     {
         CodecGemmArgs g;
-        g.a = z_;
+        g.a = w.z;
         g.lda = kCodecZ;
         g.w = qout_w_;
         g.w_f32 = qout_f32_;
@@ -332,7 +394,7 @@ void Codec::enqueue(CodecState &st, int frames, hipEvent_t *stage_ev) {
             g.M = M;
             g.N = kCodecDModel;
             g.K = S.cin;
-            g.y = y_;
+            g.y = w.y;
             g.ldy = kCodecDModel;
             ok(codec_gemm_launch(CPRO_ROWS, CEPI_STORE, g, s), "stage in");
         }
@@ -340,7 +402,7 @@ void Codec::enqueue(CodecState &st, int frames, hipEvent_t *stage_ev) {
             const int li = S.layer0 + n;
             const LayerW &L = layers_[li];
             CodecGemmArgs q;
-            q.a = y_;
+            q.a = w.y;
             q.lda = kCodecDModel;
             q.ln_w = L.n1w;
             q.ln_b = L.n1b;
@@ -349,40 +411,45 @@ void Codec::enqueue(CodecState &st, int frames, hipEvent_t *stage_ev) {
             q.M = M;
             q.N = 3 * kCodecDModel;
             q.K = kCodecDModel;
-            q.q = qb_;
+            q.q = w.qb;
             q.kc = st.k[li];
             q.vc = st.v[li];
-            q.ring = S.ring;
+            q.ring = st.ring[si];
             q.pos0 = st.pos0 + si;
-            q.freq = freq_;
+            q.rope = fa.rope[si];
             ok(codec_gemm_launch(CPRO_LN, CEPI_QKV, q, s), "qkv");
             CodecAttnArgs a;
-            a.q = qb_;
+            a.q = w.qb;
             a.kc = st.k[li];
             a.vc = st.v[li];
-            a.ring = S.ring;
+            a.ring = st.ring[si];
             a.window = S.window;
             a.M = M;
             a.splits = splits;
             a.pos0 = st.pos0 + si;
-            a.o = ao_;
-            a.st = ast_;
+            a.o = w.ao;
+            a.st = w.ast;
             ok(codec_attn_launch(a, s), "attention");
             CodecGemmArgs p;
-            p.o = ao_;
-            p.st = ast_;
-            p.splits = splits;
+            if (splits > 1) {
+                p.o = w.ao;
+                p.st = w.ast;
+                p.splits = splits;
+            } else {
+                p.a = w.ao;
+                p.lda = kCodecDModel;
+            }
             p.w = L.proj;
             p.w_f32 = L.proj_f32;
             p.M = M;
             p.N = kCodecDModel;
             p.K = kCodecDModel;
-            p.y = y_;
+            p.y = w.y;
             p.ldy = kCodecDModel;
             p.ls = L.ls1;
-            ok(codec_gemm_launch(CPRO_MERGE, CEPI_RESID, p, s), "proj");
+            ok(codec_gemm_launch(splits > 1 ? CPRO_MERGE : CPRO_ROWS, CEPI_RESID, p, s), "proj");
             CodecGemmArgs f;
-            f.a = y_;
+            f.a = w.y;
             f.lda = kCodecDModel;
             f.ln_w = L.n2w;
             f.ln_b = L.n2b;
@@ -391,25 +458,25 @@ void Codec::enqueue(CodecState &st, int frames, hipEvent_t *stage_ev) {
             f.M = M;
             f.N = L.ffn;
             f.K = kCodecDModel;
-            f.y = h_;
+            f.y = w.h;
             f.ldy = L.ffn;
             ok(codec_gemm_launch(CPRO_LN, CEPI_GELU, f, s), "f1");
             CodecGemmArgs f2;
-            f2.a = h_;
+            f2.a = w.h;
             f2.lda = L.ffn;
             f2.w = L.f2;
             f2.w_f32 = L.f2_f32;
             f2.M = M;
             f2.N = kCodecDModel;
             f2.K = L.ffn;
-            f2.y = y_;
+            f2.y = w.y;
             f2.ldy = kCodecDModel;
             f2.ls = L.ls2;
             ok(codec_gemm_launch(CPRO_ROWS, CEPI_RESID, f2, s), "f2");
         }
         {
             CodecGemmArgs g;
-            g.a = y_;
+            g.a = w.y;
             g.lda = kCodecDModel;
             g.w = S.out;
             g.w_f32 = S.out_f32;
@@ -421,7 +488,7 @@ void Codec::enqueue(CodecState &st, int frames, hipEvent_t *stage_ev) {
                 g.patch = stages_[si + 1].patch;
                 g.ldy = stages_[si + 1].cin;
             } else {  // patch 240: the samples, row-major
-                g.y = out_dev_;
+                g.y = w.out;
                 g.patch = kCodecFinalPatch;
                 g.ldy = 1;
             }
@@ -435,7 +502,7 @@ void Codec::enqueue(CodecState &st, int frames, hipEvent_t *stage_ev) {
 
 void Codec::run_piece(CodecState &st, const int32_t *codes, int frames, float *out, bool graph) {
     hipStream_t s = stream_;
-    hip_check(hipMemcpyAsync(codes_dev_, codes, sizeof(int32_t) * kCodecNq * frames, hipMemcpyHostToDevice, s),
+    hip_check(hipMemcpyAsync(work_.codes, codes, sizeof(int32_t) * kCodecNq * frames, hipMemcpyHostToDevice, s),
               "upload codes");
     if (graph) {
         auto it = graphs_.find(frames);
@@ -444,7 +511,7 @@ void Codec::run_piece(CodecState &st, const int32_t *codes, int frames, float *o
             hipGraphExec_t ge = nullptr;
             hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture");
             try {
-                enqueue(st, frames, nullptr);
+                enqueue(st, work_, work_.codes, frames, frames, nullptr);
             } catch (...) {
                 (void)hipStreamEndCapture(s, &g);
                 if (g) (void)hipGraphDestroy(g);
@@ -458,10 +525,10 @@ void Codec::run_piece(CodecState &st, const int32_t *codes, int frames, float *o
         }
         hip_check(hipGraphLaunch(it->second, s), "hipGraphLaunch");
     } else {
-        enqueue(st, frames, nullptr);
+        enqueue(st, work_, work_.codes, frames, frames, nullptr);
     }
     const size_t n = (size_t)frames * spf_;
-    hip_check(hipMemcpyAsync(out_host_, out_dev_, n * sizeof(float), hipMemcpyDeviceToHost, s), "download samples");
+    hip_check(hipMemcpyAsync(out_host_, work_.out, n * sizeof(float), hipMemcpyDeviceToHost, s), "download samples");
     hip_check(hipStreamSynchronize(s), "codec piece");
     std::memcpy(out, out_host_, n * sizeof(float));
 }
@@ -485,30 +552,36 @@ void Codec::decode(const int32_t *codes, int frames, float *out) {
     check_codes(codes, frames);
     const auto t0 = std::chrono::steady_clock::now();
     hip_check(hipSetDevice(device_), "hipSetDevice");
-    if (!whole_alloc_) {
-        alloc_state(whole_state_);
-        whole_alloc_ = true;
-    }
+    // Equal pieces, each a long run of launches: while one computes, the host copies the samples
+    // of the one before out of pinned memory.  (32-frame pieces, each waited for: 6.7 ms for 203
+    // frames, a third of it launches too small for the chip and the copy.)
+    const int pieces = (frames + kWholePiece - 1) / kWholePiece, piece = (frames + pieces - 1) / pieces;
+    ensure_whole(piece, frames);
     clear_state(whole_state_);
+    hip_check(hipMemcpyAsync(whole_work_.codes, codes, sizeof(int32_t) * kCodecNq * frames, hipMemcpyHostToDevice, stream_),
+              "upload codes");
     double stage[kCodecStages] = {0, 0, 0, 0};
-    for (int f0 = 0; f0 < frames; f0 += fmax_) {
-        const int n = std::min(fmax_, frames - f0);
-        gather_codes(codes, frames, f0, n, codes_host_);
-        hip_check(hipMemcpyAsync(codes_dev_, codes_host_, sizeof(int32_t) * kCodecNq * n, hipMemcpyHostToDevice, stream_),
-                  "upload codes");
-        hip_check(hipEventRecord(ev_[0], stream_), "hipEventRecord");
-        enqueue(whole_state_, n, ev_);
-        const size_t ns = (size_t)n * spf_;
-        hip_check(hipMemcpyAsync(out_host_, out_dev_, ns * sizeof(float), hipMemcpyDeviceToHost, stream_),
-                  "download samples");
-        hip_check(hipStreamSynchronize(stream_), "codec decode");
-        std::memcpy(out + (size_t)f0 * spf_, out_host_, ns * sizeof(float));
+    auto finish = [&](int p) {  // the samples and stage times of piece p
+        const int b = p & 1, f0 = p * piece, n = std::min(piece, frames - f0);
+        hip_check(hipEventSynchronize(done_[b]), "codec decode");
+        std::memcpy(out + (size_t)f0 * spf_, whole_host_[b], (size_t)n * spf_ * sizeof(float));
         for (int s = 0; s < kCodecStages; ++s) {
             float ms = 0.f;
-            hip_check(hipEventElapsedTime(&ms, ev_[s], ev_[s + 1]), "hipEventElapsedTime");
+            hip_check(hipEventElapsedTime(&ms, ev_[b][s], ev_[b][s + 1]), "hipEventElapsedTime");
             stage[s] += ms;
         }
+    };
+    for (int p = 0; p < pieces; ++p) {
+        const int b = p & 1, f0 = p * piece, n = std::min(piece, frames - f0);
+        hip_check(hipEventRecord(ev_[b][0], stream_), "hipEventRecord");
+        enqueue(whole_state_, whole_work_, whole_work_.codes + f0, frames, n, ev_[b]);
+        hip_check(hipMemcpyAsync(whole_host_[b], whole_work_.out, (size_t)n * spf_ * sizeof(float), hipMemcpyDeviceToHost,
+                                 stream_),
+                  "download samples");
+        hip_check(hipEventRecord(done_[b], stream_), "hipEventRecord");
+        if (p > 0) finish(p - 1);
     }
+    finish(pieces - 1);
     for (int s = 0; s < kCodecStages; ++s) stage_ms_[s] = stage[s];
     last_ms_ = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
