@@ -18,7 +18,7 @@
 // Workgroup tile: 16 rows x 16*NT columns; grid (N / (16 NT), ceil(M / 16),
 // K slices).  The 4 waves split the slice's blocks and sum in LDS; each wave
 // streams its A rows and B columns KB blocks at a time, two chunks in flight.
-#include "mh_ops.h"
+#include "mh_gemm.h"
 
 namespace mh {
 #ifdef MH_GEMM_TRACE
@@ -40,8 +40,6 @@ __device__ unsigned long long mh_gemm_ts[8192][2];
 #endif
 namespace {
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
 #ifndef MH_GEMM_KB
 #define MH_GEMM_KB 3
 #endif
@@ -49,20 +47,6 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // GEMMs (K = 768: 6 per wave, or 3 per wave in two K slices; K = 3072: 24 or 12)
 constexpr int KB = MH_GEMM_KB;
 
-
-// x = hi + lo: hi rounds toward zero (v_cvt_pkrtz, two values per
-// instruction), so x - hi is exact in fp32; lo keeps the next ~10 bits.
-__device__ __forceinline__ void split_hi_lo(const float (&x)[8], half8 &hi, half8 &lo) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const auto h = __builtin_amdgcn_cvt_pkrtz(x[2 * i], x[2 * i + 1]);
-        const auto l = __builtin_amdgcn_cvt_pkrtz(x[2 * i] - (float)h[0], x[2 * i + 1] - (float)h[1]);
-        hi[2 * i] = (_Float16)h[0];
-        hi[2 * i + 1] = (_Float16)h[1];
-        lo[2 * i] = (_Float16)l[0];
-        lo[2 * i + 1] = (_Float16)l[1];
-    }
-}
 
 // What the epilogue needs of a lane's row, computed once: a lane stores one row
 // of every column subtile of its tile.  A tile (16, 32 or 64 columns) lies inside
@@ -176,19 +160,6 @@ __device__ __forceinline__ void gemm_finish(const EpiRow &r, const EpiOps<NT> &o
     }
 }
 
-
-// Operands through buffer resources: the lane's byte offset at the wave's first
-// block is one VGPR per operand; the block within a chunk is the instruction's
-// immediate offset and the chunk base and column subtile an SGPR offset, so a
-// load costs no address arithmetic.  A load past a resource's last byte returns
-// 0 instead of faulting, so every load is unconditional (blocks past the wave's
-// last one, or rows past M, are read and never used).
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
-constexpr int kRsrcWord3 = 0x00020000;  // gfx9 raw buffer word 3 (32-bit data format)
-
-__device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, kRsrcWord3);
-}
 
 // Weights in the matrix-core order (tile_q8x4_mfma): for each 16-row subtile s
 // of W and scale block b, one 544-byte unit at (s * K/32 + b) * 544 holding the
@@ -811,6 +782,7 @@ hipError_t launch_gemm(const GemmArgs &g, Epilogue epi, KvType kv, hipStream_t s
     if (g.ln_w != nullptr && g.a_hl == nullptr &&
         (!g.ln_b || g.a8 != nullptr || epi == EPI_PART || g.K > 4 * 2 * KB * 32 || g.K < 4 * 32))
         return hipErrorInvalidValue;
+    if (tile_gemm_fits(g, epi)) return launch_gemm_tile(g, epi, kv, s);
     switch (epi) {
         case EPI_PART: return launch_a<EPI_PART, KV_F16>(g, s);
         case EPI_F32: return launch_a<EPI_F32, KV_F16>(g, s);
