@@ -83,6 +83,7 @@ private:
     float *rope_ = nullptr;                     // cos [cap+1][32] then sin
     int rope_n_ = 0;
     float *x_ = nullptr, *a_ = nullptr, *q_ = nullptr, *o_ = nullptr, *h_ = nullptr;
+    float *hidden_h_ = nullptr;  // pinned: one hidden row on its way to the caller
     float *hidden_ = nullptr, *lres_ = nullptr, *next_in_ = nullptr, *logits_ = nullptr;
     int *pos_d_ = nullptr, *codes_ = nullptr, *row_ = nullptr, *counts_ = nullptr;
     // the streams longest context first, the order of the paged attention's workgroups

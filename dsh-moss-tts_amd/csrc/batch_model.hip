@@ -104,6 +104,7 @@ Batch::Batch(Model &model, int max_streams, int capacity, KvType kv)
     hip_check(hipMemset(active_, 0, S_), "memset(active)");
     hip_check(hipMalloc(&hist_active_, (size_t)(cap_ + 1) * S_), "hipMalloc(history)");
     hip_check(hipHostMalloc(&ctrl_h_, sizeof(BatchCtl), hipHostMallocDefault), "hipHostMalloc(ctrl)");
+    hip_check(hipHostMalloc(&hidden_h_, kHidden * 4, hipHostMallocDefault), "hipHostMalloc(hidden)");
     pos_.assign(S_, 0);
 }
 
@@ -121,6 +122,7 @@ Batch::~Batch() {
     for (void *p : bufs)
         if (p) (void)hipFree(p);
     if (ctrl_h_) (void)hipHostFree(ctrl_h_);
+    if (hidden_h_) (void)hipHostFree(hidden_h_);
     if (order_h_) (void)hipHostFree(order_h_);
     if (order_) (void)hipFree(order_);
     for (auto &e : ev_)
@@ -218,18 +220,19 @@ void Batch::admit(int s, Model &src) {
     a.table_row = table_ + (size_t)s * pages_;
     a.page_size = kPage;
     a.pool_kv = kvt_;
+    a.hidden_src = v.hidden;
+    a.hidden_dst = hidden_ + (size_t)s * kHidden;
+    a.pos_dst = pos_d_ + s;
     hip_check(launch_kv_admit(a, v.pos, stream_), "kv admit");
-    hip_check(hipMemcpyAsync(hidden_ + (size_t)s * kHidden, v.hidden, kHidden * 4, hipMemcpyDeviceToDevice, stream_),
-              "hidden d2d");
-    hip_check(hipMemcpyAsync(pos_d_ + s, &v.pos, sizeof(int), hipMemcpyHostToDevice, stream_), "pos h2d");
     hip_check(hipStreamSynchronize(stream_), "sync");
     pos_[s] = v.pos;
 }
 
 void Batch::get_hidden(int s, float *out) {
     if (s < 0 || s >= S_) throw Status(MOSS_HIP_EINVAL, "stream out of range");
-    hip_check(hipMemcpyAsync(out, hidden_ + (size_t)s * kHidden, kHidden * 4, hipMemcpyDeviceToHost, stream_), "d2h");
+    hip_check(launch_row_out(hidden_ + (size_t)s * kHidden, hidden_h_, stream_), "hidden d2h");
     hip_check(hipStreamSynchronize(stream_), "sync");
+    std::memcpy(out, hidden_h_, kHidden * 4);
 }
 
 void Batch::kv_export(int s, int n_pos, float *k, float *v) {

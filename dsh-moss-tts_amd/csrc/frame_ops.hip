@@ -177,31 +177,46 @@ __global__ __launch_bounds__(256) void sample_kernel(SampleArgs a) {
     for (int c2 = t; c2 < kHidden; c2 += 256) a.next_input[c2] = q8x4_elem(a.aemb, nb, used, c2);
 }
 
+// grid (n_pos, layers, 2): position p of layer l of K (z = 0) or V (z = 1)
 template <int KV>
-__global__ void kv_import_kernel(const float *src, int n_pos, void *dst, int ctx_stride) {
+__global__ __launch_bounds__(256) void kv_import_kernel(const float *src, int n_pos, void *dst, int ctx_stride) {
     const int p = blockIdx.x;
-    for (int e = threadIdx.x; e < kHidden; e += blockDim.x) {
-        const float v = src[(size_t)p * kHidden + e];
-        const size_t idx = ((size_t)(e >> 6) * ctx_stride + p) * kHeadDim + (e & 63);
+    const size_t layer = blockIdx.z * gridDim.y + blockIdx.y;
+    const float *row = src + (layer * n_pos + p) * kHidden;
+#pragma unroll
+    for (int e = threadIdx.x; e < kHidden; e += 256) {
+        const size_t idx = ((layer * kHeads + (e >> 6)) * ctx_stride + p) * kHeadDim + (e & 63);
         if constexpr (KV == KV_F16)
-            ((__half *)dst)[idx] = __float2half_rn(v);
+            ((__half *)dst)[idx] = __float2half_rn(row[e]);
         else
-            ((float *)dst)[idx] = v;
+            ((float *)dst)[idx] = row[e];
     }
 }
 
 template <int KV>
-__global__ void kv_export_kernel(const void *src, int n_pos, int ctx_stride, float *dst) {
+__global__ __launch_bounds__(256) void kv_export_kernel(const void *src, int n_pos, int ctx_stride, float *dst) {
     const int p = blockIdx.x;
-    for (int e = threadIdx.x; e < kHidden; e += blockDim.x) {
-        const size_t idx = ((size_t)(e >> 6) * ctx_stride + p) * kHeadDim + (e & 63);
-        float v;
+    const size_t layer = blockIdx.z * gridDim.y + blockIdx.y;
+    float *row = dst + (layer * n_pos + p) * kHidden;
+#pragma unroll
+    for (int e = threadIdx.x; e < kHidden; e += 256) {
+        const size_t idx = ((layer * kHeads + (e >> 6)) * ctx_stride + p) * kHeadDim + (e & 63);
         if constexpr (KV == KV_F16)
-            v = __half2float(((const __half *)src)[idx]);
+            row[e] = __half2float(((const __half *)src)[idx]);
         else
-            v = ((const float *)src)[idx];
-        dst[(size_t)p * kHidden + e] = v;
+            row[e] = ((const float *)src)[idx];
     }
+}
+
+// grid (., runs): 16-byte words of run y
+__global__ __launch_bounds__(256) void copy_runs_kernel(const uint4 *src, size_t src_stride, uint4 *dst, size_t dst_stride,
+                                                        int words) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < words) dst[blockIdx.y * dst_stride + i] = src[blockIdx.y * src_stride + i];
+}
+
+__global__ __launch_bounds__(kHidden / 4) void row_out_kernel(const float4 *row, float4 *out) {
+    out[threadIdx.x] = row[threadIdx.x];
 }
 
 }  // namespace
@@ -246,25 +261,47 @@ hipError_t launch_sample(const SampleArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_kv_import(const float *src, int n_pos, void *dst, int ctx_stride, KvType kv, hipStream_t s) {
+hipError_t launch_kv_import(const float *src, int n_pos, void *kv_cache, int ctx_stride, KvType kv, hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
     if (n_pos <= 0) return hipSuccess;
     if (n_pos > ctx_stride) return hipErrorInvalidValue;
+    const dim3 grid(n_pos, kLayers, 2);
     if (kv == KV_F16)
-        hipLaunchKernelGGL(kv_import_kernel<KV_F16>, dim3(n_pos), dim3(256), 0, s, src, n_pos, dst, ctx_stride);
+        hipLaunchKernelGGL(kv_import_kernel<KV_F16>, grid, dim3(256), 0, s, src, n_pos, kv_cache, ctx_stride);
     else
-        hipLaunchKernelGGL(kv_import_kernel<KV_F32>, dim3(n_pos), dim3(256), 0, s, src, n_pos, dst, ctx_stride);
+        hipLaunchKernelGGL(kv_import_kernel<KV_F32>, grid, dim3(256), 0, s, src, n_pos, kv_cache, ctx_stride);
     return hipGetLastError();
 }
 
-hipError_t launch_kv_export(const void *src, int n_pos, int ctx_stride, KvType kv, float *dst, hipStream_t s) {
+hipError_t launch_kv_export(const void *kv_cache, int n_pos, int ctx_stride, KvType kv, float *dst, hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
     if (n_pos <= 0) return hipSuccess;
     if (n_pos > ctx_stride) return hipErrorInvalidValue;
+    const dim3 grid(n_pos, kLayers, 2);
     if (kv == KV_F16)
-        hipLaunchKernelGGL(kv_export_kernel<KV_F16>, dim3(n_pos), dim3(256), 0, s, src, n_pos, ctx_stride, dst);
+        hipLaunchKernelGGL(kv_export_kernel<KV_F16>, grid, dim3(256), 0, s, kv_cache, n_pos, ctx_stride, dst);
     else
-        hipLaunchKernelGGL(kv_export_kernel<KV_F32>, dim3(n_pos), dim3(256), 0, s, src, n_pos, ctx_stride, dst);
+        hipLaunchKernelGGL(kv_export_kernel<KV_F32>, grid, dim3(256), 0, s, kv_cache, n_pos, ctx_stride, dst);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_runs(const void *src, size_t src_stride, void *dst, size_t dst_stride, size_t bytes, int runs,
+                            hipStream_t s) {
+    (void)hipGetLastError();  // report only this launch's error, not a stale one
+    if (bytes == 0 || runs <= 0) return hipSuccess;
+    if ((src_stride | dst_stride | bytes | (size_t)(uintptr_t)src | (size_t)(uintptr_t)dst) % 16 || bytes / 16 > INT32_MAX ||
+        runs > 65535)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(copy_runs_kernel, dim3((unsigned)((bytes / 16 + 255) / 256), runs), dim3(256), 0, s,
+                       static_cast<const uint4 *>(src), src_stride / 16, static_cast<uint4 *>(dst), dst_stride / 16,
+                       (int)(bytes / 16));
+    return hipGetLastError();
+}
+
+hipError_t launch_row_out(const float *row, float *out, hipStream_t s) {
+    (void)hipGetLastError();  // report only this launch's error, not a stale one
+    hipLaunchKernelGGL(row_out_kernel, dim3(1), dim3(kHidden / 4), 0, s, reinterpret_cast<const float4 *>(row),
+                       reinterpret_cast<float4 *>(out));
     return hipGetLastError();
 }
 
@@ -708,28 +745,44 @@ __global__ void kv_export_paged_kernel(const void *pool, const int *table_row, i
     }
 }
 
-// grid (n_pos, layers, 2): position p of layer l of K (z = 0) or V (z = 1); thread t copies
-// element t of the 768 (head t / 64, dim t % 64) and t + 256, t + 512.
+// grid (pages, heads, 2 layers): a workgroup moves one head's positions of one page, a run of
+// 64-value rows on both sides, 8 values a thread; workgroup 0 also takes the hidden state and the
+// position.  One launch where four transfers ran per admission (8-byte and 3 KB copies each as
+// long as the keys): 20.5 -> 15 us a call for 65 to 200 positions.
 template <int SK, int DK>
-__global__ __launch_bounds__(256) void kv_admit_kernel(KvAdmit a) {
-    const int p = blockIdx.x, l = blockIdx.y, z = blockIdx.z;
+__global__ __launch_bounds__(256) void kv_admit_kernel(KvAdmit a, int n_pos) {
+    const int pg = blockIdx.x, h = blockIdx.y, l = blockIdx.z >> 1, z = blockIdx.z & 1;
+    if ((blockIdx.x | blockIdx.y | blockIdx.z) == 0) {
+        if (threadIdx.x < kHidden / 4)
+            reinterpret_cast<float4 *>(a.hidden_dst)[threadIdx.x] = reinterpret_cast<const float4 *>(a.hidden_src)[threadIdx.x];
+        if (threadIdx.x == 255) *a.pos_dst = n_pos;
+    }
+    const int p0 = pg * a.page_size, n = min(a.page_size, n_pos - p0) * (kHeadDim / 8);  // (none when n_pos is 0)
+    constexpr int SB = SK == KV_F16 ? 2 : 4, DB = DK == KV_F16 ? 2 : 4;
     const uint8_t *src = static_cast<const uint8_t *>(z ? a.v_src : a.k_src) +
-                         (size_t)l * a.src_layer_elems * (SK == KV_F16 ? 2 : 4);
-    uint8_t *pool = static_cast<uint8_t *>(z ? a.v_pool : a.k_pool) + (size_t)l * a.pool_layer_elems * (DK == KV_F16 ? 2 : 4);
-    const size_t page_base = (size_t)a.table_row[p / a.page_size] * kHeads * a.page_size;
-    for (int e = threadIdx.x; e < kHidden; e += blockDim.x) {
-        const int h = e >> 6, d = e & 63;
-        const size_t si = ((size_t)h * a.ctx_stride + p) * kHeadDim + d;
-        const size_t di = ((page_base + (size_t)h * a.page_size) + p % a.page_size) * kHeadDim + d;
+                         ((size_t)l * a.src_layer_elems + ((size_t)h * a.ctx_stride + p0) * kHeadDim) * SB;
+    uint8_t *dst = static_cast<uint8_t *>(z ? a.v_pool : a.k_pool) +
+                   ((size_t)l * a.pool_layer_elems + ((size_t)a.table_row[pg] * kHeads + h) * a.page_size * kHeadDim) * DB;
+    for (int i = threadIdx.x; i < n; i += 256) {
         if constexpr (SK == DK) {
-            if constexpr (SK == KV_F16)
-                ((__half *)pool)[di] = ((const __half *)src)[si];
-            else
-                ((float *)pool)[di] = ((const float *)src)[si];
+#pragma unroll
+            for (int w = 0; w < SB / 2; ++w)
+                reinterpret_cast<uint4 *>(dst)[(SB / 2) * i + w] = reinterpret_cast<const uint4 *>(src)[(SB / 2) * i + w];
         } else if constexpr (SK == KV_F32) {
-            ((__half *)pool)[di] = __float2half_rn(((const float *)src)[si]);
+            const float *x = reinterpret_cast<const float *>(src) + 8 * i;
+            uint32_t u[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[e] = (uint32_t)f2h(x[2 * e]) | (uint32_t)f2h(x[2 * e + 1]) << 16;
+            reinterpret_cast<uint4 *>(dst)[i] = make_uint4(u[0], u[1], u[2], u[3]);
         } else {
-            ((float *)pool)[di] = __half2float(((const __half *)src)[si]);
+            const uint4 v = reinterpret_cast<const uint4 *>(src)[i];
+            const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+            float *y = reinterpret_cast<float *>(dst) + 8 * i;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                y[2 * e] = h2f((uint16_t)u[e]);
+                y[2 * e + 1] = h2f((uint16_t)(u[e] >> 16));
+            }
         }
     }
 }
@@ -738,22 +791,17 @@ __global__ __launch_bounds__(256) void kv_admit_kernel(KvAdmit a) {
 
 hipError_t launch_kv_admit(const KvAdmit &a, int n_pos, hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
-    if (n_pos <= 0) return hipSuccess;
-    if (!a.k_src || !a.v_src || !a.k_pool || !a.v_pool || !a.table_row || a.page_size <= 0 || n_pos > a.ctx_stride)
+    if (!a.k_src || !a.v_src || !a.k_pool || !a.v_pool || !a.table_row || !a.hidden_src || !a.hidden_dst || !a.pos_dst ||
+        a.page_size <= 0 || n_pos < 0 || n_pos > a.ctx_stride)
         return hipErrorInvalidValue;
-    const dim3 grid(n_pos, kLayers, 2);
-    if (a.src_kv == KV_F16) {
-        if (a.pool_kv == KV_F16)
-            hipLaunchKernelGGL((kv_admit_kernel<KV_F16, KV_F16>), grid, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((kv_admit_kernel<KV_F16, KV_F32>), grid, dim3(256), 0, s, a);
-    } else {
-        if (a.pool_kv == KV_F16)
-            hipLaunchKernelGGL((kv_admit_kernel<KV_F32, KV_F16>), grid, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((kv_admit_kernel<KV_F32, KV_F32>), grid, dim3(256), 0, s, a);
-    }
-    return hipGetLastError();
+    const dim3 grid(n_pos > 0 ? (n_pos + a.page_size - 1) / a.page_size : 1, kHeads, 2 * kLayers);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a, n_pos);
+        return hipGetLastError();
+    };
+    if (a.src_kv == KV_F16)
+        return a.pool_kv == KV_F16 ? go(kv_admit_kernel<KV_F16, KV_F16>) : go(kv_admit_kernel<KV_F16, KV_F32>);
+    return a.pool_kv == KV_F16 ? go(kv_admit_kernel<KV_F32, KV_F16>) : go(kv_admit_kernel<KV_F32, KV_F32>);
 }
 
 hipError_t launch_kv_import_paged(const float *src, int n_pos, void *pool, const int *table_row, int page_size,

@@ -146,6 +146,7 @@ private:
     void launch_frame_local(hipStream_t s, bool text_gate, bool fused);
     void write_state_header();
     void *kv_layer(int which, int layer) const;  // which: 0 = K, 1 = V
+    float *kv_stage(int n_pos);
 
     int device_ = 0, max_ctx_ = kMaxCtx, use_graphs_ = 1;
     bool prefill_a16_ = false;  // prefill GEMMs on fp32 activations (else W8A8)
@@ -190,6 +191,10 @@ private:
     float *lkv_ = nullptr;               // [2][heads][17][64] fp32
     float *rope_ = nullptr;              // cos [n][32] then sin [n][32]
     int rope_n_ = 0;
+    float *hidden_h_ = nullptr;  // pinned: the hidden row on its way to the caller
+    float *logits_h_ = nullptr;  // pinned: [2 readback slots][16][1024], when a caller takes logits
+    float *kv_stage_ = nullptr;  // kv_export / kv_import
+    size_t kv_stage_n_ = 0;      // its floats
     float *x_ = nullptr, *q_ = nullptr, *mlp_ = nullptr, *hidden_ = nullptr;
     float *lres_ = nullptr, *next_in_ = nullptr, *slot_in_ = nullptr;
     float *attn_out_ = nullptr;

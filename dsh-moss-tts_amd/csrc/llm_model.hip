@@ -222,6 +222,7 @@ Model::Model(const void *blob, size_t bytes, const moss_hip_llm_options &opt) {
     hip_check(hipMalloc(&state_, sizeof(DevState)), "hipMalloc(state)");
     hip_check(hipHostMalloc(&hstate_, sizeof(DevState), hipHostMallocDefault), "hipHostMalloc(state)");
     hip_check(hipHostMalloc(&hread_, 2 * sizeof(DevState), hipHostMallocDefault), "hipHostMalloc(state readback)");
+    hip_check(hipHostMalloc(&hidden_h_, kHidden * 4, hipHostMallocDefault), "hipHostMalloc(hidden)");
     std::memset(hstate_, 0, sizeof(DevState));
     hstate_->rep_penalty = 1.0f;
     hip_check(hipMemcpy(state_, hstate_, sizeof(DevState), hipMemcpyHostToDevice), "init state");
@@ -273,11 +274,13 @@ Model::~Model() {
     if (g_global_) (void)hipGraphExecDestroy(g_global_);
     if (g_local_) (void)hipGraphExecDestroy(g_local_);
     if (g_local_fused_) (void)hipGraphExecDestroy(g_local_fused_);
-    void *bufs[] = {blob_, wm_, kv_, lkv_, rope_, x_, q_, mlp_, hidden_, lres_, next_in_, slot_in_, attn_out_, attn_part_, pre_x_, pre_a_, pre_q_, pre_h_, pre_part_, pre_q8_, pre_d8_, pre_q8h_, pre_d8h_, logits_, counts_, forced_, text_logits_, rows_dev_, state_, snap_, ll_, qkv_table_, layer_args_, cap_dec_, cap_pre_};
+    void *bufs[] = {blob_, wm_, kv_, lkv_, rope_, x_, q_, mlp_, hidden_, lres_, next_in_, slot_in_, attn_out_, attn_part_, pre_x_, pre_a_, pre_q_, pre_h_, pre_part_, pre_q8_, pre_d8_, pre_q8h_, pre_d8h_, logits_, counts_, forced_, text_logits_, rows_dev_, state_, snap_, ll_, qkv_table_, layer_args_, cap_dec_, cap_pre_, kv_stage_};
     for (void *p : bufs)
         if (p) (void)hipFree(p);
     if (hstate_) (void)hipHostFree(hstate_);
     if (hread_) (void)hipHostFree(hread_);
+    if (hidden_h_) (void)hipHostFree(hidden_h_);
+    if (logits_h_) (void)hipHostFree(logits_h_);
     for (auto &e : ev_)
         if (e) (void)hipEventDestroy(e);
     if (stream_) (void)hipStreamDestroy(stream_);
@@ -615,8 +618,9 @@ size_t Model::capture_read(int what, void *out, size_t bytes) {
 }
 
 void Model::get_hidden(float *out) {
-    hip_check(hipMemcpyAsync(out, hidden_, kHidden * 4, hipMemcpyDeviceToHost, stream_), "hidden d2h");
+    hip_check(launch_row_out(hidden_, hidden_h_, stream_), "hidden d2h");
     hip_check(hipStreamSynchronize(stream_), "sync");
+    std::memcpy(out, hidden_h_, kHidden * 4);
 }
 
 void Model::set_hidden(const float *in) {
@@ -899,6 +903,11 @@ int Model::generate(int max_frames, const moss_hip_sample_params &p, uint64_t se
     // does, and a cancel flag raised there stops the loop before frame f + 1.
     // A G(f) enqueued behind an L(f) that the end gate stopped is a no-op on the
     // device (every kernel tests state->stop first); the host does not count it.
+    // A frame's logits go to the caller through pinned slots like the state: copied straight to
+    // pageable memory, a frame's launches waited for its copy (65 KB, 13 us a frame).
+    if (logits_dump && !logits_h_)
+        hip_check(hipHostMalloc(&logits_h_, 2 * sizeof(float) * kNVq * kCodebook, hipHostMallocDefault),
+                  "hipHostMalloc(logits)");
     bool global_enq[2] = {false, false};
     int pos_next = pos_;  // position once every enqueued global step has run
     auto enqueue = [&](int f) {
@@ -908,7 +917,7 @@ int Model::generate(int max_frames, const moss_hip_sample_params &p, uint64_t se
         launch_frame_local(stream_, gate_dump != nullptr, hstate_->cfg.greedy != 0);
         if (timing) hip_check(hipEventRecord(ev[kEvLocal1], stream_), "event");
         if (logits_dump)
-            hip_check(hipMemcpyAsync(logits_dump + (size_t)f * kNVq * kCodebook, logits_,
+            hip_check(hipMemcpyAsync(logits_h_ + (size_t)slot * kNVq * kCodebook, logits_,
                                      sizeof(float) * kNVq * kCodebook, hipMemcpyDeviceToHost, stream_),
                       "logits d2h");
         hip_check(hipMemcpyAsync(hread_ + slot, state_, sizeof(DevState), hipMemcpyDeviceToHost, stream_),
@@ -976,6 +985,9 @@ int Model::generate(int max_frames, const moss_hip_sample_params &p, uint64_t se
             hstate_->ll_err = hs.ll_err;
             check_exchange();
             if (timing && f > 0) frame_timing(f - 1);  // G(f - 1) ran before L(f)
+            if (logits_dump)
+                std::memcpy(logits_dump + (size_t)f * kNVq * kCodebook, logits_h_ + (size_t)slot * kNVq * kCodebook,
+                            sizeof(float) * kNVq * kCodebook);
             if (gate_dump) {
                 float *gd = gate_dump + 4 * (size_t)f;
                 gd[0] = hs.gate[0];
@@ -1025,13 +1037,9 @@ void Model::snapshot_prefix() {
     if (prefix_pos_ <= 0) return;
     const size_t width = (size_t)prefix_pos_ * kHeadDim * kv_esize_;
     hip_check(hipMalloc(&snap_, 2ull * kLayers * kHeads * width), "hipMalloc(snapshot)");
-    for (int w = 0; w < 2; ++w)
-        for (int l = 0; l < kLayers; ++l) {
-            uint8_t *dst = static_cast<uint8_t *>(snap_) + ((size_t)w * kLayers + l) * kHeads * width;
-            hip_check(hipMemcpy2DAsync(dst, width, kv_layer(w, l), (size_t)max_ctx_ * kHeadDim * kv_esize_, width,
-                                       kHeads, hipMemcpyDeviceToDevice, stream_),
-                      "snapshot copy");
-        }
+    hip_check(launch_copy_runs(kv_, (size_t)max_ctx_ * kHeadDim * kv_esize_, snap_, width, width, 2 * kLayers * kHeads,
+                               stream_),
+              "snapshot copy");
     hip_check(hipStreamSynchronize(stream_), "sync");
 }
 
@@ -1041,59 +1049,47 @@ void Model::restore_prefix() {
         return;
     }
     const size_t width = (size_t)prefix_pos_ * kHeadDim * kv_esize_;
-    for (int w = 0; w < 2; ++w)
-        for (int l = 0; l < kLayers; ++l) {
-            const uint8_t *src = static_cast<const uint8_t *>(snap_) + ((size_t)w * kLayers + l) * kHeads * width;
-            hip_check(hipMemcpy2DAsync(kv_layer(w, l), (size_t)max_ctx_ * kHeadDim * kv_esize_, src, width, width,
-                                       kHeads, hipMemcpyDeviceToDevice, stream_),
-                      "restore copy");
-        }
+    hip_check(launch_copy_runs(snap_, width, kv_, (size_t)max_ctx_ * kHeadDim * kv_esize_, width, 2 * kLayers * kHeads,
+                               stream_),
+              "restore copy");
     hip_check(hipStreamSynchronize(stream_), "sync");
     pos_ = prefix_pos_;
+}
+
+// The fp32 rows of n_pos positions of every layer's K and V, between kv_export / kv_import and
+// the caller's memory; grown to the largest call.
+float *Model::kv_stage(int n_pos) {
+    const size_t need = 2 * (size_t)kLayers * n_pos * kHidden;
+    if (need > kv_stage_n_) {
+        if (kv_stage_) hip_check(hipFree(kv_stage_), "free stage");
+        kv_stage_ = nullptr;
+        kv_stage_n_ = 0;
+        hip_check(hipMalloc(&kv_stage_, need * 4), "hipMalloc(stage)");
+        kv_stage_n_ = need;
+    }
+    return kv_stage_;
 }
 
 void Model::kv_export(int n_pos, float *k, float *v) {
     if (n_pos < 0 || n_pos > max_ctx_) throw Status(MOSS_HIP_EINVAL, "n_pos out of range");
     if (n_pos == 0) return;
-    float *stage = nullptr;
-    const size_t per = (size_t)n_pos * kHidden;
-    hip_check(hipMalloc(&stage, per * 4), "hipMalloc(stage)");
-    try {
-        for (int w = 0; w < 2; ++w)
-            for (int l = 0; l < kLayers; ++l) {
-                hip_check(launch_kv_export(kv_layer(w, l), n_pos, max_ctx_, kvt_, stage, stream_), "kv export");
-                hip_check(hipMemcpyAsync((w == 0 ? k : v) + (size_t)l * per, stage, per * 4, hipMemcpyDeviceToHost,
-                                         stream_),
-                          "kv d2h");
-                hip_check(hipStreamSynchronize(stream_), "sync");
-            }
-    } catch (...) {
-        (void)hipFree(stage);
-        throw;
-    }
-    (void)hipFree(stage);
+    const size_t per = (size_t)kLayers * n_pos * kHidden;
+    float *stage = kv_stage(n_pos);
+    hip_check(launch_kv_export(kv_, n_pos, max_ctx_, kvt_, stage, stream_), "kv export");
+    hip_check(hipMemcpyAsync(k, stage, per * 4, hipMemcpyDeviceToHost, stream_), "kv d2h");
+    hip_check(hipMemcpyAsync(v, stage + per, per * 4, hipMemcpyDeviceToHost, stream_), "kv d2h");
+    hip_check(hipStreamSynchronize(stream_), "sync");
 }
 
 void Model::kv_import(int n_pos, const float *k, const float *v, const float *hidden) {
     if (n_pos < 0 || n_pos > max_ctx_) throw Status(MOSS_HIP_EINVAL, "n_pos out of range");
-    float *stage = nullptr;
-    const size_t per = (size_t)n_pos * kHidden;
     if (n_pos > 0) {
-        hip_check(hipMalloc(&stage, per * 4), "hipMalloc(stage)");
-        try {
-            for (int w = 0; w < 2; ++w)
-                for (int l = 0; l < kLayers; ++l) {
-                    hip_check(hipMemcpyAsync(stage, (w == 0 ? k : v) + (size_t)l * per, per * 4, hipMemcpyHostToDevice,
-                                             stream_),
-                              "kv h2d");
-                    hip_check(launch_kv_import(stage, n_pos, kv_layer(w, l), max_ctx_, kvt_, stream_), "kv import");
-                    hip_check(hipStreamSynchronize(stream_), "sync");
-                }
-        } catch (...) {
-            (void)hipFree(stage);
-            throw;
-        }
-        (void)hipFree(stage);
+        const size_t per = (size_t)kLayers * n_pos * kHidden;
+        float *stage = kv_stage(n_pos);
+        hip_check(hipMemcpyAsync(stage, k, per * 4, hipMemcpyHostToDevice, stream_), "kv h2d");
+        hip_check(hipMemcpyAsync(stage + per, v, per * 4, hipMemcpyHostToDevice, stream_), "kv h2d");
+        hip_check(launch_kv_import(stage, n_pos, kv_, max_ctx_, kvt_, stream_), "kv import");
+        hip_check(hipStreamSynchronize(stream_), "sync");
     }
     if (hidden) set_hidden(hidden);
     pos_ = n_pos;

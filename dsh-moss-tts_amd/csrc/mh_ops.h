@@ -367,15 +367,21 @@ hipError_t launch_local_qkv_rows(const LocalQkv &a, int streams, hipStream_t s);
 // pos[s] += 1 for active streams; streams reaching capacity become inactive.
 hipError_t launch_advance_rows(const StreamState &st, int streams, hipStream_t s);
 
-// KV import/export between the reference layout [n][768] fp32 of one layer and the
-// device layout [heads][ctx_stride][64] (fp16 or fp32).
-hipError_t launch_kv_import(const float *src, int n_pos, void *dst, int ctx_stride, KvType kv, hipStream_t s);
+// KV import/export of every layer between the reference layout, K then V as [layer][n][768]
+// fp32, and the device cache [K, V][layer][heads][ctx_stride][64] (fp16 or fp32).
+hipError_t launch_kv_import(const float *src, int n_pos, void *kv_cache, int ctx_stride, KvType kv, hipStream_t s);
 // Same into pages: position p -> page table_row[p / page_size], slot p % page_size of [page][head][page_size][64].
 hipError_t launch_kv_import_paged(const float *src, int n_pos, void *pool, const int *table_row, int page_size,
                                   KvType kv, hipStream_t s);
 hipError_t launch_kv_export_paged(const void *pool, const int *table_row, int page_size, int n_pos, KvType kv,
                                   float *dst, hipStream_t s);
-hipError_t launch_kv_export(const void *src, int n_pos, int ctx_stride, KvType kv, float *dst, hipStream_t s);
+hipError_t launch_kv_export(const void *kv_cache, int n_pos, int ctx_stride, KvType kv, float *dst, hipStream_t s);
+// `runs` runs of `bytes`, each stride bytes after the one before (all multiples of 16).
+hipError_t launch_copy_runs(const void *src, size_t src_stride, void *dst, size_t dst_stride, size_t bytes, int runs,
+                            hipStream_t s);
+// A row of 768 floats to host memory that the device can write (pinned): a 3 KB copy through
+// the runtime takes three times as long as this launch.
+hipError_t launch_row_out(const float *row, float *out, hipStream_t s);
 // Device to device, every layer's K and V: positions [0, n_pos) of a contiguous cache
 // ([layer][head][ctx_stride][64], layer l of K at k_src + l * src_layer_elems) into the pages
 // of one stream (layer l of K at k_pool + l * pool_layer_elems), converted from src_kv to
@@ -390,6 +396,9 @@ struct KvAdmit {
     const int *table_row = nullptr;
     int page_size = 0;
     KvType pool_kv = KV_F16;
+    const float *hidden_src = nullptr;  // [768], to hidden_dst
+    float *hidden_dst = nullptr;
+    int *pos_dst = nullptr;  // takes n_pos
 };
 hipError_t launch_kv_admit(const KvAdmit &a, int n_pos, hipStream_t s);
 
