@@ -315,9 +315,10 @@ __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, 
         lds_barrier();
     }
 
-    // sums of 64 columns at a time, then those (one chain over K = 1024 measured twice the error
-    // of the sums split over waves, 7e-7 against 4e-7 after all layers)
-    floatx4 acc[MT][NT], tot[MT][NT];
+    // sums of 64 columns at a time in two chains (even and odd columns), then those: the chains
+    // of the 16 x 16 tile's waves are no longer (one chain over K = 1024 measured twice their
+    // error after all layers, 7e-7 against 4e-7, one chain per 64 columns 4.4e-7)
+    floatx4 acc[2][MT][NT], tot[MT][NT];
     auto clear = [](floatx4 (&v)[MT][NT]) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -328,10 +329,12 @@ __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, 
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) tot[i][j] += acc[i][j];
-        clear(acc);
+            for (int j = 0; j < NT; ++j) tot[i][j] += acc[0][i][j] + acc[1][i][j];
+        clear(acc[0]);
+        clear(acc[1]);
     };
-    clear(acc);
+    clear(acc[0]);
+    clear(acc[1]);
     clear(tot);
     auto step = [&](int s, int kk) {
         float a[MT][8];
@@ -360,7 +363,7 @@ __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, 
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = mfma4(a[i][k], wr[s][j].get(k), acc[i][j]);
+                for (int j = 0; j < NT; ++j) acc[k & 1][i][j] = mfma4(a[i][k], wr[s][j].get(k), acc[k & 1][i][j]);
     };
     int kk = 0;
     for (; kk + 64 <= g.K; kk += 64) {
@@ -404,10 +407,27 @@ __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, 
 //   S^T = K Q^T: A = K[key kb + l%16][16g + t], B = Q[q l%16][16g + t], t = 0..15
 //   O^T = V^T P^T per 4-column group j: A = V[key kb + 4g + s][4(l%16) + j], B = P[q][kb + 4g + s]
 // so the lane with q = l%16 holds S^T for keys kb + 4g + i and O for columns 16g..16g+15.
+//
+// Many unsplit tiles (XCD) are a linear grid: workgroups go to the 8 XCDs in turn and within one to
+// its 32 CUs in turn, so an XCD works on every other tile of one head, whose keys its L2 keeps, and
+// its tiles go out longest first (an utterance's first rows see few keys), every other round of
+// 32 backwards, so that a CU which drew a long tile draws a short one next.
+// With two register sets for the keys in turn and no division a key, a 203-frame utterance spends
+// 0.80 ms here, 1.13 before.
+template <bool XCD>
 __global__ __launch_bounds__(256) void codec_attn_kernel(const CodecAttnArgs a) {
     __shared__ float red[4][16 * 64 + 32];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, col = lane & 15, grp = lane >> 4;
-    const int m0 = blockIdx.x * 16, h = blockIdx.y, split = blockIdx.z;
+    int tile = blockIdx.x, h = blockIdx.y;
+    if constexpr (XCD) {
+        const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3, n = gridDim.x >> 3;
+        const int row = at >> 5, in_row = min(32, n - 32 * row);
+        const int rank = 32 * row + ((row & 1) ? in_row - 1 - (at & 31) : at & 31);
+        h = xcd >> 1;
+        tile = ((a.M + 15) >> 4) - 1 - 2 * rank - (xcd & 1);
+        if (tile < 0) return;  // uniform (an odd number of tiles)
+    }
+    const int m0 = tile * 16, split = blockIdx.z;
     const int P0 = *a.pos0;
     const int mlast = min(m0 + 15, a.M - 1);
     const int klo = max(0, P0 + m0 - a.window + 1), khi = P0 + mlast;
@@ -436,37 +456,29 @@ __global__ __launch_bounds__(256) void codec_attn_kernel(const CodecAttnArgs a) 
     for (int j = 0; j < 4; ++j) o[j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     // block b's operands: K rows kb + l%16 (this lane's 16 columns of the head), V rows
-    // kb + 4g + s (4 columns); keys past khi read as zeros (their scores are masked)
+    // kb + 4g + s (4 columns); keys past khi read as key khi (their scores are masked)
+    // the ring slot of key klo + i (i < ring: the ring holds the window and the piece)
+    const int slot0 = klo % a.ring, span = khi - klo;
+    auto slot = [&](int i) {
+        const int s = slot0 + min(i, span);
+        return (size_t)(s < a.ring ? s : s - a.ring) * kCodecDModel;
+    };
     auto load_block = [&](int b, float (&kv)[16], float4 (&vv)[4]) {
-        const int kb = klo + 16 * b;
-        const int kp = kb + col;
-        const bool ok = kp <= khi;
-        const float4 *src = reinterpret_cast<const float4 *>(a.kc + (size_t)((ok ? kp : klo) % a.ring) * kCodecDModel + hoff + 16 * grp);
+        const float4 *src = reinterpret_cast<const float4 *>(a.kc + slot(16 * b + col) + hoff + 16 * grp);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float4 v = ok ? src[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float4 v = src[i];
             kv[4 * i] = v.x;
             kv[4 * i + 1] = v.y;
             kv[4 * i + 2] = v.z;
             kv[4 * i + 3] = v.w;
         }
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int kq = kb + 4 * grp + s;
-            vv[s] = kq <= khi ? *reinterpret_cast<const float4 *>(a.vc + (size_t)(kq % a.ring) * kCodecDModel + hoff + 4 * col)
-                              : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+        for (int s = 0; s < 4; ++s)
+            vv[s] = *reinterpret_cast<const float4 *>(a.vc + slot(16 * b + 4 * grp + s) + hoff + 4 * col);
     };
-    float kv[16];
-    float4 vv[4];
-    if (b0 + wave < b1) load_block(b0 + wave, kv, vv);
-    for (int b = b0 + wave; b < b1; b += 4) {
+    auto block = [&](int b, const float (&kv)[16], const float4 (&vv)[4]) {
         const int kb = klo + 16 * b;
-        // the wave's next block is in flight while this one is computed
-        float kn[16];
-        float4 vn[4];
-        const bool more = b + 4 < b1;
-        if (more) load_block(b + 4, kn, vn);
         floatx4 sc0 = {0.f, 0.f, 0.f, 0.f}, sc1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
@@ -500,12 +512,18 @@ __global__ __launch_bounds__(256) void codec_attn_kernel(const CodecAttnArgs a) 
             o[2] = mfma4(vv[s].z, p[s], o[2]);
             o[3] = mfma4(vv[s].w, p[s], o[3]);
         }
-        if (more) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) kv[i] = kn[i];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) vv[i] = vn[i];
-        }
+    };
+    // the wave's next block is in flight while one is computed, in the other of two register
+    // sets; a request past the last block reads the last key again
+    float k0[16], k1[16];
+    float4 v0[4], v1[4];
+    if (b0 + wave < b1) load_block(b0 + wave, k0, v0);
+    for (int b = b0 + wave; b < b1; b += 8) {
+        load_block(b + 4, k1, v1);
+        block(b, k0, v0);
+        if (b + 4 >= b1) break;
+        load_block(b + 8, k0, v0);
+        block(b + 4, k1, v1);
     }
     lrun += xshfl<16>(lrun);
     lrun += xshfl<32>(lrun);
@@ -665,8 +683,12 @@ int codec_attn_launch(const CodecAttnArgs &a, hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
     if (a.M <= 0 || a.splits < 1 || a.window <= 0 || a.ring <= 0 || !a.q || !a.kc || !a.vc || !a.pos0 || !a.o || !a.st)
         return MOSS_HIP_EINVAL;
-    const dim3 grid((a.M + 15) / 16, kCodecHeads, a.splits);
-    hipLaunchKernelGGL(codec_attn_kernel, grid, dim3(256), 0, s, a);
+    const int tiles = (a.M + 15) / 16;
+    static_assert(kCodecHeads == 4, "two XCDs a head");
+    if (a.splits == 1 && tiles * kCodecHeads > 256)  // more than one workgroup per CU
+        hipLaunchKernelGGL(codec_attn_kernel<true>, dim3(8 * ((tiles + 1) / 2)), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL(codec_attn_kernel<false>, dim3(tiles, kCodecHeads, a.splits), dim3(256), 0, s, a);
     return hipGetLastError() == hipSuccess ? 0 : MOSS_HIP_EDEVICE;
 }
 
