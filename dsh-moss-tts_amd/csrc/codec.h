@@ -31,7 +31,7 @@ constexpr int kCodecDModel = 256, kCodecHeads = 4, kCodecHeadDim = 64;
 constexpr int kCodecNq = 16, kCodecCb = 1024, kCodecCbDim = 8, kCodecZ = 512;
 constexpr int kCodecStages = 4;
 constexpr int kCodecFinalPatch = 240;
-constexpr int kCodecMaxSplits = 12;  // key splits of an attention launch (its merge holds them all in registers)
+constexpr int kCodecMaxSplits = 4;   // key splits of an attention launch (its merge holds them all in registers)
 
 // Activation source of a codec GEMM (staged into LDS as fp32, 16 rows at a time).
 enum CodecPro : int {

@@ -56,32 +56,51 @@ struct W8 {
     }
 };
 
-// RoPE of a QKV column: pairs (2i, 2i+1), angle = float(pos) * freq in fp32 (audio_rope,
-// audio_layer.cpp:30-44), cos and sin from the piece's table; q to its buffer, k and v to the
-// ring slot of the row's position.
-__device__ __forceinline__ void qkv_store(const CodecGemmArgs &g, int m, int nn, float v, float partner) {
-    const int region = nn / kCodecDModel, c = nn - region * kCodecDModel;
-    float out = v;
-    if (region < 2) {
-        const float2 cs = g.rope[(size_t)m * (kCodecHeadDim / 2) + ((c & (kCodecHeadDim - 1)) >> 1)];
-        out = (c & 1) ? partner * cs.y + v * cs.x : v * cs.x - partner * cs.y;
-    }
-    float *dst = region == 0 ? g.q : (region == 1 ? g.kc : g.vc);
-    const size_t row = region == 0 ? (size_t)m : (size_t)((*g.pos0 + m) % g.ring);
-    dst[row * kCodecDModel + c] = out;
-}
+// What element (m, nn) of a product needs besides its sum, loaded before any element is stored:
+// a load behind a store that may alias it costs its own round trip (QKV in large tiles 28.5 ->
+// 23.8 us a launch of an utterance, f2 and proj 22.5 -> 20.7; in an 8-frame chunk, with the
+// operands requested first of all, QKV 7.4 -> 6.7, f1 6.3 -> 5.8).
+struct EpiIn {
+    float2 cs;       // CEPI_QKV: cos and sin of the element's RoPE pair
+    float *out;      // CEPI_QKV: where it goes
+    float y, ls, b;  // CEPI_RESID: the residual and its layer scale; CEPI_STORE: the bias
+};
 
 template <int EPI>
-__device__ __forceinline__ void epi_store(const CodecGemmArgs &g, int m, int nn, float v) {
-    if constexpr (EPI == CEPI_STORE) {
+__device__ __forceinline__ EpiIn epi_load(const CodecGemmArgs &g, int m, int nn) {
+    EpiIn e;
+    if constexpr (EPI == CEPI_QKV) {
+        // q to its buffer, k and v to the ring slot of the row's position; cos and sin from the
+        // piece's table (loaded for v too: no branch)
+        const int region = nn / kCodecDModel, c = nn - region * kCodecDModel;
+        const int slot = (*g.pos0 + m) % g.ring;
+        float *dst = region == 0 ? g.q : (region == 1 ? g.kc : g.vc);
+        e.out = dst + (size_t)(region == 0 ? m : slot) * kCodecDModel + c;
+        e.cs = g.rope[(size_t)m * (kCodecHeadDim / 2) + ((c & (kCodecHeadDim - 1)) >> 1)];
+    } else if constexpr (EPI == CEPI_RESID) {
+        e.y = g.y[(size_t)m * g.ldy + nn];
+        e.ls = g.ls[nn];
+    } else if constexpr (EPI == CEPI_STORE) {
+        e.b = g.bias ? g.bias[nn] : 0.f;
+    }
+    return e;
+}
+
+// partner: the sum of column nn ^ 1 of the row (CEPI_QKV: interleaved RoPE, audio_layer.cpp:30-44)
+template <int EPI>
+__device__ __forceinline__ void epi_store(const CodecGemmArgs &g, const EpiIn &e, int m, int nn, float v, float partner) {
+    if constexpr (EPI == CEPI_QKV) {
+        float out = v;
+        if (nn < 2 * kCodecDModel) out = (nn & 1) ? partner * e.cs.y + v * e.cs.x : v * e.cs.x - partner * e.cs.y;
+        *e.out = out;
+    } else if constexpr (EPI == CEPI_STORE) {
         const int p = g.patch;
-        g.y[((size_t)m * p + nn % p) * g.ldy + nn / p] = g.bias ? v + g.bias[nn] : v;
+        g.y[((size_t)m * p + nn % p) * g.ldy + nn / p] = g.bias ? v + e.b : v;
     } else if constexpr (EPI == CEPI_GELU) {
         // audio_gelu (audio_layer.cpp:46)
         g.y[(size_t)m * g.ldy + nn] = 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
     } else {
-        float *y = g.y + (size_t)m * g.ldy + nn;
-        *y = *y + g.ls[nn] * v;
+        g.y[(size_t)m * g.ldy + nn] = e.y + e.ls * v;
     }
 }
 
@@ -92,7 +111,9 @@ __device__ __forceinline__ void epi_store(const CodecGemmArgs &g, int m, int nn,
 // flight before the first MFMA); the 4 partial tiles are summed in LDS and thread t
 // finishes element (t / 16, t % 16).  Prologues transform A as it is loaded:
 // CPRO_LN with per-row (mean, 1/std) from LDS, CPRO_MERGE with wave w = head w.
-constexpr int kWaveChunks = 8;  // chunks of 32 per wave per round (rounds of 1024 columns)
+// chunks of 32 per wave per round: rounds of 1024 columns, or all of K = 256 under a prologue
+template <int PRO>
+constexpr int kWaveChunks = PRO == CPRO_ROWS ? 8 : 2;
 
 template <int PRO, int EPI, int WF32>
 __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) {
@@ -103,6 +124,9 @@ __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) 
     const int am = m0 + col;        // A row this lane feeds
     const bool avalid = am < g.M;
     const int n = n0 + col;          // W row this lane feeds (N % 16 == 0: always valid)
+    constexpr int WC = kWaveChunks<PRO>;
+    const int fm = m0 + (t >> 4), fn = n0 + (t & 15);  // the element this thread finishes
+    const EpiIn ein = epi_load<EPI>(g, min(fm, g.M - 1), fn);
 
     // CPRO_MERGE: this lane's (row am, head = wave) split weights e^(m_s - M) / sum_s e^(m_s - M) l_s.
     // Every split's statistics are loaded before any is used (a loop over the splits waited for
@@ -126,13 +150,13 @@ __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) 
     }
 
     floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < g.K; k0 += 32 * 4 * kWaveChunks) {
-        const int nch = min(4 * kWaveChunks, (g.K - k0) >> 5);
+    for (int k0 = 0; k0 < g.K; k0 += 32 * 4 * WC) {
+        const int nch = min(4 * WC, (g.K - k0) >> 5);
         const int c0 = wave * nch / 4, c1 = (wave + 1) * nch / 4;
-        float4 av[kWaveChunks][2];
-        W8<WF32> wr[kWaveChunks];
+        float4 av[WC][2];
+        W8<WF32> wr[WC];
 #pragma unroll
-        for (int c = 0; c < kWaveChunks; ++c) {
+        for (int c = 0; c < WC; ++c) {
             const int kk = k0 + 32 * (c0 + c) + 8 * grp;
             if (c0 + c < c1) {
                 wr[c].load(g.w, (size_t)n * g.K + kk);
@@ -170,7 +194,19 @@ __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) 
                 av[c][0] = av[c][1] = make_float4(0.f, 0.f, 0.f, 0.f);
             }
         }
-        if constexpr (PRO == CPRO_LN) {  // K == 256: one round; the loads above are in flight
+        float lw[PRO == CPRO_LN ? WC : 1][8], lb[PRO == CPRO_LN ? WC : 1][8];
+        if constexpr (PRO == CPRO_LN) {  // K == 256: one round of two chunks a wave; the loads above are in flight
+#pragma unroll
+            for (int c = 0; c < WC; ++c) {
+                const float4 *wp = reinterpret_cast<const float4 *>(g.ln_w + 32 * (c0 + c) + 8 * grp);
+                const float4 *bp = reinterpret_cast<const float4 *>(g.ln_b + 32 * (c0 + c) + 8 * grp);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const float4 w = wp[i], b = bp[i];
+                    lw[c][4 * i] = w.x, lw[c][4 * i + 1] = w.y, lw[c][4 * i + 2] = w.z, lw[c][4 * i + 3] = w.w;
+                    lb[c][4 * i] = b.x, lb[c][4 * i + 1] = b.y, lb[c][4 * i + 2] = b.z, lb[c][4 * i + 3] = b.w;
+                }
+            }
             // audio_layernorm (audio_layer.cpp:17-28): two-pass mean / variance over 256, eps 1e-5
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -185,24 +221,17 @@ __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) 
                     rowst[r] = make_float2(0.f, 0.f);
                 }
             }
-            __syncthreads();
+            lds_barrier();
         }
 #pragma unroll
-        for (int c = 0; c < kWaveChunks; ++c) {
+        for (int c = 0; c < WC; ++c) {
             if (c0 + c < c1) {
                 float a[8] = {av[c][0].x, av[c][0].y, av[c][0].z, av[c][0].w,
                               av[c][1].x, av[c][1].y, av[c][1].z, av[c][1].w};
                 if constexpr (PRO == CPRO_LN) {
-                    const int kk = k0 + 32 * (c0 + c) + 8 * grp;
                     const float2 rs = rowst[col];
-                    const float4 w0 = *reinterpret_cast<const float4 *>(g.ln_w + kk);
-                    const float4 w1 = *reinterpret_cast<const float4 *>(g.ln_w + kk + 4);
-                    const float4 b0 = *reinterpret_cast<const float4 *>(g.ln_b + kk);
-                    const float4 b1 = *reinterpret_cast<const float4 *>(g.ln_b + kk + 4);
-                    const float lw[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-                    const float lb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) a[i] = avalid ? (a[i] - rs.x) * rs.y * lw[i] + lb[i] : 0.f;
+                    for (int i = 0; i < 8; ++i) a[i] = avalid ? (a[i] - rs.x) * rs.y * lw[c][i] + lb[c][i] : 0.f;
                 } else if constexpr (PRO == CPRO_MERGE) {
 #pragma unroll
                     for (int i = 0; i < 8; ++i) a[i] *= inv_den;
@@ -221,17 +250,14 @@ __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) 
     const floatx4 acc = acc0 + acc1;
 #pragma unroll
     for (int i = 0; i < 4; ++i) red[wave][(4 * grp + i) * 16 + col] = acc[i];
-    __syncthreads();
-    const int r = t >> 4, cn = t & 15, m = m0 + r, nn = n0 + cn;
+    lds_barrier();
     const float v = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
-    if (m >= g.M) return;
-
+    float partner = 0.f;
     if constexpr (EPI == CEPI_QKV) {
         const int tp = t ^ 1;
-        qkv_store(g, m, nn, v, (red[0][tp] + red[1][tp]) + (red[2][tp] + red[3][tp]));
-    } else {
-        epi_store<EPI>(g, m, nn, v);
+        partner = (red[0][tp] + red[1][tp]) + (red[2][tp] + red[3][tp]);
     }
+    if (fm < g.M) epi_store<EPI>(g, ein, fm, fn, v, partner);
 }
 
 // The same product for pieces with many rows: a workgroup takes 32 MT rows x 32 NT columns,
@@ -378,6 +404,14 @@ __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, 
         flush();
     }
 
+    EpiIn ein[MT][4][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                ein[i][e][j] = epi_load<EPI>(g, min(m0 + wm + 16 * i + 4 * grp + e, g.M - 1), min(wn + 16 * j + col, g.N - 1));
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -387,12 +421,8 @@ __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, 
             for (int j = 0; j < NT; ++j) {
                 const int nn = wn + 16 * j + col;
                 const float v = tot[i][j][e];
-                if constexpr (EPI == CEPI_QKV) {
-                    const float partner = xshfl<1>(v);
-                    if (m < g.M && nn < g.N) qkv_store(g, m, nn, v, partner);
-                } else {
-                    if (m < g.M && nn < g.N) epi_store<EPI>(g, m, nn, v);
-                }
+                const float partner = EPI == CEPI_QKV ? xshfl<1>(v) : 0.f;
+                if (m < g.M && nn < g.N) epi_store<EPI>(g, ein[i][e][j], m, nn, v, partner);
             }
         }
 }
@@ -400,7 +430,7 @@ __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, 
 // Windowed causal attention of 16 query rows x one head over the ring's keys
 // (attention_window_avx2, attn_avx2.cpp:93-204): key position kp is visible to the
 // query at position qp iff 0 <= qp - kp < window.  Grid (row tiles, heads, splits):
-// split z takes a contiguous share of the tile's 16-key blocks, its 4 waves every 4th
+// split z takes a contiguous share of the tile's 16-key blocks, its WV waves every WVth
 // block of it, each with a running max / sum (online softmax); the waves merge in LDS
 // and the split writes its unnormalised output and (max, sum) for the proj GEMM's
 // merge prologue.
@@ -414,9 +444,9 @@ __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, 
 // 32 backwards, so that a CU which drew a long tile draws a short one next.
 // With two register sets for the keys in turn and no division a key, a 203-frame utterance spends
 // 0.80 ms here, 1.13 before.
-template <bool XCD>
-__global__ __launch_bounds__(256) void codec_attn_kernel(const CodecAttnArgs a) {
-    __shared__ float red[4][16 * 64 + 32];
+template <int WV, bool XCD>
+__global__ __launch_bounds__(64 * WV) void codec_attn_kernel(const CodecAttnArgs a) {
+    __shared__ float red[WV][16 * 64 + 32];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, col = lane & 15, grp = lane >> 4;
     int tile = blockIdx.x, h = blockIdx.y;
     if constexpr (XCD) {
@@ -518,12 +548,12 @@ __global__ __launch_bounds__(256) void codec_attn_kernel(const CodecAttnArgs a) 
     float k0[16], k1[16];
     float4 v0[4], v1[4];
     if (b0 + wave < b1) load_block(b0 + wave, k0, v0);
-    for (int b = b0 + wave; b < b1; b += 8) {
-        load_block(b + 4, k1, v1);
+    for (int b = b0 + wave; b < b1; b += 2 * WV) {
+        load_block(b + WV, k1, v1);
         block(b, k0, v0);
-        if (b + 4 >= b1) break;
-        load_block(b + 8, k0, v0);
-        block(b + 4, k1, v1);
+        if (b + WV >= b1) break;
+        load_block(b + 2 * WV, k0, v0);
+        block(b + WV, k1, v1);
     }
     lrun += xshfl<16>(lrun);
     lrun += xshfl<32>(lrun);
@@ -537,29 +567,34 @@ __global__ __launch_bounds__(256) void codec_attn_kernel(const CodecAttnArgs a) 
         R[1024 + col] = mrun;
         R[1040 + col] = lrun;
     }
-    __syncthreads();
-    const int q = t >> 4, d4 = t & 15, m = m0 + q;
+    lds_barrier();
+    constexpr int E = 16 / WV;  // columns a thread finishes, of row t % 16
+    const int q = t & 15, d = E * (t >> 4), m = m0 + q;
     if (m >= a.M) return;
     float mx = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) mx = fmaxf(mx, red[w][1024 + q]);
+    for (int w = 0; w < WV; ++w) mx = fmaxf(mx, red[w][1024 + q]);
     const float msafe = mx == -INFINITY ? 0.f : mx;
-    float l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
+    float l = 0.f, acc[E] = {};
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < WV; ++w) {
         const float f = exp_f(red[w][1024 + q] - msafe);
         l += f * red[w][1040 + q];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] += f * red[w][(4 * d4 + e) * 16 + q];
+        for (int e = 0; e < E; ++e) acc[e] += f * red[w][(d + e) * 16 + q];
     }
     if (a.splits == 1) {
         const float inv = 1.0f / l;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] *= inv;
+        for (int e = 0; e < E; ++e) acc[e] *= inv;
     }
     const size_t row = (size_t)split * a.M + m;
-    *reinterpret_cast<float4 *>(a.o + row * kCodecDModel + hoff + 4 * d4) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    if (d4 == 0 && a.splits > 1) a.st[row * kCodecHeads + h] = make_float2(mx, l);
+    float *out = a.o + row * kCodecDModel + hoff + d;
+    if constexpr (E == 4)
+        *reinterpret_cast<float4 *>(out) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    else
+        *reinterpret_cast<float2 *>(out) = make_float2(acc[0], acc[1]);
+    if (d == 0 && a.splits > 1) a.st[row * kCodecHeads + h] = make_float2(mx, l);
 }
 
 // Workgroup t < frames: z[t][r] = sum_i (b_i[r] + sum_k W_i[r][k] cb_i[code_it][k]), i in order
@@ -686,9 +721,9 @@ int codec_attn_launch(const CodecAttnArgs &a, hipStream_t s) {
     const int tiles = (a.M + 15) / 16;
     static_assert(kCodecHeads == 4, "two XCDs a head");
     if (a.splits == 1 && tiles * kCodecHeads > 256)  // more than one workgroup per CU
-        hipLaunchKernelGGL(codec_attn_kernel<true>, dim3(8 * ((tiles + 1) / 2)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((codec_attn_kernel<4, true>), dim3(8 * ((tiles + 1) / 2)), dim3(256), 0, s, a);
     else
-        hipLaunchKernelGGL(codec_attn_kernel<false>, dim3(tiles, kCodecHeads, a.splits), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((codec_attn_kernel<8, false>), dim3(tiles, kCodecHeads, a.splits), dim3(512), 0, s, a);
     return hipGetLastError() == hipSuccess ? 0 : MOSS_HIP_EDEVICE;
 }
 

@@ -220,15 +220,15 @@ Codec::~Codec() {
     if (stream_) (void)hipStreamDestroy(stream_);
 }
 
-// Key splits of a stage's attention for a piece of `rows` rows: enough workgroups to
-// cover the chip (~512 = row tiles x 4 heads x splits), each split keeping >= 8 key
-// blocks of 16 (two per wave) of the steady-state window.  (More splits, ~2048
-// workgroups, measured no faster and cost the proj GEMM's merge more.)
+// Key splits of a stage's attention for a piece of `rows` rows: enough workgroups (row tiles x
+// 4 heads x splits, of 8 waves) for one per CU, each split keeping >= 16 key blocks of 16 (two per
+// wave) of the steady-state window.  Every column tile of proj merges all splits of its rows
+// again, so twice as many splits of 4 waves made proj of an 8-frame chunk 8.4 us a launch where it is 5.2 now.
 int Codec::splits_for(int stage, int rows) const {
     const int tiles = (rows + 15) / 16;
     const int blocks = (stages_[stage].window + 15 + 15) / 16;
-    const int want = (512 + tiles * kCodecHeads - 1) / (tiles * kCodecHeads);
-    return std::max(1, std::min(std::min(want, blocks / 8), kCodecMaxSplits));
+    const int want = (256 + tiles * kCodecHeads - 1) / (tiles * kCodecHeads);
+    return std::max(1, std::min(std::min(want, blocks / 16), kCodecMaxSplits));
 }
 
 // Buffers for pieces of up to `frames` frames.
