@@ -313,22 +313,29 @@ __device__ __forceinline__ void mfma_chunk(const Chunk<NT, A8, AT> &c, int b0, i
 // per-16-column (mean, M2) pairs (GemmArgs::ln_stats), combined in a fixed order (Chan
 // et al.'s pairwise update; every merge is symmetric in its two sides, so all lanes
 // agree); ln_w / ln_b are staged in lw2 / lb2.  Returns (mean, 1 / sqrt(var + eps)) of
-// row m_base + l16 after one barrier.
-__device__ __forceinline__ float2 ln_rows_from_stats(const GemmArgs &g, int m_base, int l16, float *lw2, float *lb2,
-                                                     float2 *rstat) {
+// row m_base + l16 after one barrier, which orders LDS only: the operands' loads stay in
+// flight.  The statistics are requested before those (StatsIn): loads return in order.
+struct StatsIn {
+    float2 p[3];
+    float lw[3], lb[3];
+    __device__ __forceinline__ void load(const GemmArgs &g, int m_base) {
+        const int tr = threadIdx.x >> 4, sub = threadIdx.x & 15;
+        const int sr = min(m_base + tr, g.M - 1);
+        const float2 *ps = reinterpret_cast<const float2 *>(g.ln_stats);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) p[i] = ps[(size_t)(3 * sub + i) * g.M + sr];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            lw[i] = g.ln_w[threadIdx.x + 256 * i];
+            lb[i] = g.ln_b[threadIdx.x + 256 * i];
+        }
+    }
+};
+
+__device__ __forceinline__ float2 ln_rows_from_stats(const StatsIn &in, int l16, float *lw2, float *lb2, float2 *rstat) {
 #pragma clang fp contract(off)
     const int tr = threadIdx.x >> 4, sub = threadIdx.x & 15;
-    const int sr = min(m_base + tr, g.M - 1);
-    const float2 *ps = reinterpret_cast<const float2 *>(g.ln_stats);
-    float2 p[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) p[i] = ps[(size_t)(3 * sub + i) * g.M + sr];
-    float lw[3], lb[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        lw[i] = g.ln_w[threadIdx.x + 256 * i];
-        lb[i] = g.ln_b[threadIdx.x + 256 * i];
-    }
+    const float2(&p)[3] = in.p;
     // groups 3 sub .. 3 sub + 2 (16 columns each), then the 16 lanes of the row
     float mean = p[0].x, m2 = p[0].y;
     {
@@ -352,11 +359,11 @@ __device__ __forceinline__ float2 ln_rows_from_stats(const GemmArgs &g, int m_ba
     }
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-        lw2[threadIdx.x + 256 * i] = lw[i];
-        lb2[threadIdx.x + 256 * i] = lb[i];
+        lw2[threadIdx.x + 256 * i] = in.lw[i];
+        lb2[threadIdx.x + 256 * i] = in.lb[i];
     }
     if (sub == 0) rstat[tr] = make_float2(mean, 1.0f / sqrtf(m2 / (float)kHidden + 1e-5f));
-    __syncthreads();
+    lds_barrier();
     return rstat[l16];
 }
 
@@ -436,9 +443,12 @@ __global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
         // measured slower than either.)
         __shared__ float lnw2[kHidden], lnb2[kHidden];
         __shared__ float2 rstat[16];
+        StatsIn si;
+        si.load(g, m_base);
         Chunk<NT, A8, AT> ca, cb;
-        if (nb > 0) load_chunk<NT, A8, TL, AT>(ca, 0, src);
-        const float2 st = ln_rows_from_stats(g, m_base, l16, lnw2, lnb2, rstat);
+        load_chunk<NT, A8, TL, AT>(ca, 0, src);
+        load_chunk<NT, A8, TL, AT>(cb, KB, src);
+        const float2 st = ln_rows_from_stats(si, l16, lnw2, lnb2, rstat);
         const float mean = st.x, inv = st.y;
         auto ln_apply = [&](Chunk<NT, A8, AT> &c, int b0) {  // columns 32 blk + 8 kq + i
 #pragma unroll
@@ -455,15 +465,11 @@ __global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
                     split_hi_lo(x, c.xh[j], c.xl[j]);
                 }
         };
-        for (int b0 = 0; b0 < nb; b0 += 2 * KB) {
-            load_chunk<NT, A8, TL, AT>(cb, b0 + KB, src);
-            ln_apply(ca, b0);
-            mfma_chunk<NT, A8, AT>(ca, b0, nb, kq, acc);
-            if (b0 + KB >= nb) break;
-            if (b0 + 2 * KB < nb) load_chunk<NT, A8, TL, AT>(ca, b0 + 2 * KB, src);
-            ln_apply(cb, b0 + KB);
-            mfma_chunk<NT, A8, AT>(cb, b0 + KB, nb, kq, acc);
-        }
+        static_assert(4 * 2 * KB * 32 == kHidden, "K = 768: a wave has two chunks, both in flight");
+        ln_apply(ca, 0);
+        mfma_chunk<NT, A8, AT>(ca, 0, nb, kq, acc);
+        ln_apply(cb, KB);
+        mfma_chunk<NT, A8, AT>(cb, KB, nb, kq, acc);
     } else if constexpr (LN && !AT) {
         __shared__ float lnw[4 * 2 * KB * 32], lnb[4 * 2 * KB * 32];
         __shared__ float lsum[4][16], lsq[4][16];
