@@ -20,6 +20,8 @@
 // streams its A rows and B columns KB blocks at a time, two chunks in flight.
 #include "mh_gemm.h"
 
+#include <type_traits>
+
 namespace mh {
 #ifdef MH_GEMM_TRACE
 // Start and end time (100 MHz device clock) of every workgroup of the last
@@ -312,9 +314,8 @@ __device__ __forceinline__ void mfma_chunk(const Chunk<NT, A8, AT> &c, int b0, i
 // LayerNorm row statistics of a workgroup's 16 rows (K = 768) from a producer's
 // per-16-column (mean, M2) pairs (GemmArgs::ln_stats), combined in a fixed order (Chan
 // et al.'s pairwise update; every merge is symmetric in its two sides, so all lanes
-// agree); ln_w / ln_b are staged in lw2 / lb2.  Returns (mean, 1 / sqrt(var + eps)) of
-// row m_base + l16 after one barrier, which orders LDS only: the operands' loads stay in
-// flight.  The statistics are requested before those (StatsIn): loads return in order.
+// agree); ln_w / ln_b are staged in lw2 / lb2, (mean, 1 / sqrt(var + eps)) of the rows in
+// rstat.  The barrier that follows orders LDS only: the operands' loads stay in flight.  The statistics are requested before those (StatsIn): loads return in order.
 struct StatsIn {
     float2 p[3];
     float lw[3], lb[3];
@@ -332,7 +333,7 @@ struct StatsIn {
     }
 };
 
-__device__ __forceinline__ float2 ln_rows_from_stats(const StatsIn &in, int l16, float *lw2, float *lb2, float2 *rstat) {
+__device__ __forceinline__ void ln_rows_from_stats(const StatsIn &in, float *lw2, float *lb2, float2 *rstat) {
 #pragma clang fp contract(off)
     const int tr = threadIdx.x >> 4, sub = threadIdx.x & 15;
     const float2(&p)[3] = in.p;
@@ -363,16 +364,18 @@ __device__ __forceinline__ float2 ln_rows_from_stats(const StatsIn &in, int l16,
         lb2[threadIdx.x + 256 * i] = in.lb[i];
     }
     if (sub == 0) rstat[tr] = make_float2(mean, 1.0f / sqrtf(m2 / (float)kHidden + 1e-5f));
-    lds_barrier();
-    return rstat[l16];
 }
 
-// WV: waves per workgroup, 4, or 8 for a long K with the residual epilogue (fc_out, K = 3072:
+// WV: waves per workgroup, 4, or 8 under LN of pre-split rows (3 blocks a wave, then summed in wave
+// order) and for a long K with the residual epilogue (fc_out, K = 3072:
 // 12 blocks per wave, so the sum needs no second kernel); waves 4..7 only contribute partials.
 template <int EPI, int KV, int NT, bool A8, bool LN, bool TL, bool AT, int WV = 4>
 __global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
 #pragma clang fp contract(off)
-    static_assert(WV == 4 || (WV == 8 && EPI == EPI_RESID && !LN), "8 waves: the residual epilogue only");
+    static_assert(WV == 4 || (WV == 8 && ((LN && AT) || (EPI == EPI_RESID && !LN))), "8 waves: LN of pre-split rows, or a residual");
+    // 8 waves: both halves of them finish, each its half of the column subtiles if there are two
+    constexpr bool kSplitFin = WV == 8 && NT >= 2;
+    constexpr int FT = kSplitFin ? NT / 2 : NT;
     GT_START
     __shared__ floatx4 red[WV][NT][64];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -390,9 +393,10 @@ __global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
     // the epilogue: wave w finishes row 4kq + w of every column subtile; its operands
     // are requested first (loads complete in order, so these never delay the operands')
     const int erow = m_base + 4 * kq + (wave & 3);
+    const int t0 = kSplitFin ? (wave >> 2) * FT : 0;  // the first subtile it finishes
     const EpiRow er = epi_row<EPI, KV>(g, erow, n_base);
-    EpiOps<NT> eo;
-    epi_load<EPI, NT>(g, er, n_base, l16, eo);
+    EpiOps<FT> eo;
+    epi_load<EPI, FT>(g, er, n_base + 16 * t0, l16, eo);
     Src<A8> src;
     {
         const uint32_t a_elems = (uint32_t)((g.M - 1) * g.lda + g.K);
@@ -444,11 +448,13 @@ __global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
         __shared__ float lnw2[kHidden], lnb2[kHidden];
         __shared__ float2 rstat[16];
         StatsIn si;
-        si.load(g, m_base);
+        if (wave < 4) si.load(g, m_base);  // (uniform) 256 threads merge the statistics
         Chunk<NT, A8, AT> ca, cb;
         load_chunk<NT, A8, TL, AT>(ca, 0, src);
-        load_chunk<NT, A8, TL, AT>(cb, KB, src);
-        const float2 st = ln_rows_from_stats(si, l16, lnw2, lnb2, rstat);
+        if constexpr (WV == 4) load_chunk<NT, A8, TL, AT>(cb, KB, src);
+        if (wave < 4) ln_rows_from_stats(si, lnw2, lnb2, rstat);
+        lds_barrier();
+        const float2 st = rstat[l16];
         const float mean = st.x, inv = st.y;
         auto ln_apply = [&](Chunk<NT, A8, AT> &c, int b0) {  // columns 32 blk + 8 kq + i
 #pragma unroll
@@ -465,11 +471,13 @@ __global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
                     split_hi_lo(x, c.xh[j], c.xl[j]);
                 }
         };
-        static_assert(4 * 2 * KB * 32 == kHidden, "K = 768: a wave has two chunks, both in flight");
+        static_assert(4 * 2 * KB * 32 == kHidden, "K = 768: a wave of 4 has two chunks, both in flight");
         ln_apply(ca, 0);
         mfma_chunk<NT, A8, AT>(ca, 0, nb, kq, acc);
-        ln_apply(cb, KB);
-        mfma_chunk<NT, A8, AT>(cb, KB, nb, kq, acc);
+        if constexpr (WV == 4) {
+            ln_apply(cb, KB);
+            mfma_chunk<NT, A8, AT>(cb, KB, nb, kq, acc);
+        }
     } else if constexpr (LN && !AT) {
         __shared__ float lnw[4 * 2 * KB * 32], lnb[4 * 2 * KB * 32];
         __shared__ float lsum[4][16], lsq[4][16];
@@ -569,7 +577,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
     for (int t = 0; t < NT; ++t) red[wave][t][lane] = acc[t];
     __syncthreads();
     // lane holds rows m_base + 4kq + i, column n_base + 16t + l16
-    if constexpr (EPI == EPI_GELU && NT >= 2) {
+    if constexpr (EPI == EPI_GELU && NT >= 2 && WV == 4) {
         if (g.q8_out != nullptr) {  // uniform
             // wave w finishes row 4kq + w of every subtile: a 32-block is subtiles (2b, 2b + 1)
             // across the 16 lanes of a kq group, so its amax is a 16-lane reduction
@@ -610,19 +618,19 @@ __global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
             return;
         }
     }
-    if (WV > 4 && wave >= 4) return;  // (uniform) their partials are in LDS
+    if (WV > 4 && !kSplitFin && wave >= 4) return;  // (uniform) their partials are in LDS
     // component w of each lane's partials: one 4-byte LDS read each, at an offset
     // uniform in the wave; the waves' partials summed in wave order
-    const int i = wave, m = erow;
+    const int i = wave & 3, m = erow;
     const float *redf = (const float *)&red[0][0][lane] + i;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        float v = redf[4 * (t * 64)];
+    for (int t = 0; t < FT; ++t) {
+        float v = redf[4 * ((t0 + t) * 64)];
 #pragma unroll
-        for (int w = 1; w < WV; ++w) v += redf[4 * ((w * NT + t) * 64)];
-        const int n = n_base + 16 * t + l16;
+        for (int w = 1; w < WV; ++w) v += redf[4 * ((w * NT + t0 + t) * 64)];
+        const int n = n_base + 16 * (t0 + t) + l16;
         const float partner = xshfl<1>(v);  // column n ^ 1, same row
-        if (m < g.M) gemm_finish<EPI, KV, NT>(er, eo, t, n, v, partner);
+        if (m < g.M) gemm_finish<EPI, KV, FT>(er, eo, t, n, v, partner);
         if constexpr (EPI == EPI_F32) {
             if (g.pick_pairs != nullptr) {  // uniform: the 16 lanes of a row hold 16 consecutive columns
                 float best = -INFINITY;
@@ -674,7 +682,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
                 q += xshfl<4>(q);
                 q += xshfl<8>(q);
                 if (l16 == 0 && m < g.M)
-                    reinterpret_cast<float2 *>(g.y_stats)[(size_t)((n_base >> 4) + t) * g.M + m] = make_float2(mean, q);
+                    reinterpret_cast<float2 *>(g.y_stats)[(size_t)((n_base >> 4) + t0 + t) * g.M + m] = make_float2(mean, q);
             }
         }
     }
@@ -699,14 +707,27 @@ hipError_t launch_nt(const GemmArgs &g, hipStream_t s) {
     const int kz = EPI == EPI_PART ? (g.ksplit > 0 ? g.ksplit : gemm_ksplit(g.M, g.N, g.K)) : 1;
     // the widest column tile that still gives ~192 workgroups (a quantising epilogue needs
     // whole 32-blocks in a tile: at least 32 columns)
-    if (g.N % 64 == 0 && (g.N / 64) * mt * kz >= 192) {
-        hipLaunchKernelGGL((gemm_wk_kernel<EPI, KV, 4, A8, LN, TL, AT>), dim3(g.N / 64, mt, kz), dim3(256), 0, s, g);
-    } else if (g.N % 32 == 0 && ((g.N / 32) * mt * kz >= 192 || g.q8_out != nullptr)) {
-        hipLaunchKernelGGL((gemm_wk_kernel<EPI, KV, 2, A8, LN, TL, AT>), dim3(g.N / 32, mt, kz), dim3(256), 0, s, g);
-    } else {
-        hipLaunchKernelGGL((gemm_wk_kernel<EPI, KV, 1, A8, LN, TL, AT>), dim3(g.N / 16, mt, kz), dim3(256), 0, s, g);
-    }
-    return hipGetLastError();
+    const int nt = g.N % 64 == 0 && (g.N / 64) * mt * kz >= 192                              ? 4
+                   : g.N % 32 == 0 && ((g.N / 32) * mt * kz >= 192 || g.q8_out != nullptr) ? 2
+                                                                                           : 1;
+    auto go = [&](auto n, auto wv) {
+        constexpr int NT = decltype(n)::value, WV = decltype(wv)::value;
+        hipLaunchKernelGGL((gemm_wk_kernel<EPI, KV, NT, A8, LN, TL, AT, WV>), dim3(g.N / (16 * NT), mt, kz), dim3(64 * WV),
+                           0, s, g);
+        return hipGetLastError();
+    };
+    auto go_nt = [&](auto wv) {
+        return nt == 4   ? go(std::integral_constant<int, 4>(), wv)
+               : nt == 2 ? go(std::integral_constant<int, 2>(), wv)
+                         : go(std::integral_constant<int, 1>(), wv);
+    };
+    // with a LayerNorm to apply to pre-split rows, 8 waves: normalising is half of a wave's work
+    // (M = 64 / 128, 4 and 8 waves: fc_in 8.1 / 11.0 and 6.8 / 10.0 us, QKV 8.3 / 10.0 and 7.9 / 9.4,
+    // a head 5.8 / 7.0 and 5.4 / 6.0; without one the second set of waves only adds partial sums:
+    // fc_in 6.5 and 7.0, proj 4.1 and 4.9)
+    constexpr int WV = LN && AT ? 8 : 4;
+    if (WV == 8 && g.q8_out != nullptr) return hipErrorInvalidValue;  // (its halves finish apart)
+    return go_nt(std::integral_constant<int, WV>());
 }
 
 template <int EPI, int KV, bool TL>
