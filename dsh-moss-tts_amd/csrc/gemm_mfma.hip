@@ -370,7 +370,7 @@ __device__ __forceinline__ void ln_rows_from_stats(const StatsIn &in, float *lw2
 // order) and for a long K with the residual epilogue (fc_out, K = 3072:
 // 12 blocks per wave, so the sum needs no second kernel); waves 4..7 only contribute partials.
 template <int EPI, int KV, int NT, bool A8, bool LN, bool TL, bool AT, int WV = 4>
-__global__ __launch_bounds__(64 * WV) void gemm_wk_kernel(GemmArgs g) {
+__global__ __launch_bounds__(64 * WV, WV == 8 && EPI == EPI_RESID && NT == 2 ? 4 : 1) void gemm_wk_kernel(GemmArgs g) {
 #pragma clang fp contract(off)
     static_assert(WV == 4 || (WV == 8 && ((LN && AT) || (EPI == EPI_RESID && !LN))), "8 waves: LN of pre-split rows, or a residual");
     // 8 waves: both halves of them finish, each its half of the column subtiles if there are two
@@ -694,13 +694,17 @@ hipError_t launch_nt(const GemmArgs &g, hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
     const int mt = (g.M + 15) / 16;
     if constexpr (EPI == EPI_RESID && !LN) {
-        // a long K (fc_out, K = 3072) in one workgroup of 8 waves, 16 columns a tile: each wave
-        // takes 12 blocks (4 chunks of 3) and the residual epilogue completes the rows (no
-        // split-K reduce) (32-column tiles, half the workgroups: 64 streams 56.4k -> 54.4k
-        // frames/s; 16 waves of 6 blocks: 56.66k -> 56.59k)
+        // a long K (fc_out, K = 3072) in one workgroup of 8 waves: each wave takes 12 blocks (4 chunks
+        // of 3) and the residual epilogue completes the rows (no split-K reduce; 16 waves of 6
+        // blocks: 56.66k -> 56.59k frames/s).  Tiles of 16 columns up to one workgroup per CU, of
+        // 32 beyond (64, 96, 160, 201 rows, 16 and 32 columns: 6.8, 8.6, 9.6, 12.0 and 7.2, 7.5, 7.9,
+        // 11.4 us); at most 128 VGPRs, so that two fit a CU
         if (g.K >= 2048) {
-            hipLaunchKernelGGL((gemm_wk_kernel<EPI, KV, 1, A8, LN, TL, AT, 8>), dim3(g.N / 16, mt, 1), dim3(512), 0, s,
-                               g);
+            if (g.N % 32 == 0 && (g.N / 16) * mt > 256)
+                hipLaunchKernelGGL((gemm_wk_kernel<EPI, KV, 2, A8, LN, TL, AT, 8>), dim3(g.N / 32, mt, 1), dim3(512), 0, s, g);
+            else
+                hipLaunchKernelGGL((gemm_wk_kernel<EPI, KV, 1, A8, LN, TL, AT, 8>), dim3(g.N / 16, mt, 1), dim3(512), 0, s,
+                                   g);
             return hipGetLastError();
         }
     }
