@@ -215,6 +215,15 @@ __global__ __launch_bounds__(256) void copy_runs_kernel(const uint4 *src, size_t
     if (i < words) dst[blockIdx.y * dst_stride + i] = src[blockIdx.y * src_stride + i];
 }
 
+static_assert(sizeof(DevState) % 4 == 0 && sizeof(DevState) <= 4 * 256, "one word a thread");
+__global__ __launch_bounds__(256) void frame_out_kernel(const DevState *state, DevState *state_out, const float4 *logits,
+                                                        float4 *logits_out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < (int)(sizeof(DevState) / 4))
+        reinterpret_cast<uint32_t *>(state_out)[i] = reinterpret_cast<const uint32_t *>(state)[i];
+    if (logits != nullptr) logits_out[i] = logits[i];
+}
+
 __global__ __launch_bounds__(kHidden / 4) void row_out_kernel(const float4 *row, float4 *out) {
     out[threadIdx.x] = row[threadIdx.x];
 }
@@ -295,6 +304,14 @@ hipError_t launch_copy_runs(const void *src, size_t src_stride, void *dst, size_
     hipLaunchKernelGGL(copy_runs_kernel, dim3((unsigned)((bytes / 16 + 255) / 256), runs), dim3(256), 0, s,
                        static_cast<const uint4 *>(src), src_stride / 16, static_cast<uint4 *>(dst), dst_stride / 16,
                        (int)(bytes / 16));
+    return hipGetLastError();
+}
+
+hipError_t launch_frame_out(const DevState *state, DevState *state_out, const float *logits, float *logits_out,
+                            hipStream_t s) {
+    (void)hipGetLastError();  // report only this launch's error, not a stale one
+    hipLaunchKernelGGL(frame_out_kernel, dim3(logits ? kNVq * kCodebook / 4 / 256 : 1), dim3(256), 0, s, state, state_out,
+                       reinterpret_cast<const float4 *>(logits), reinterpret_cast<float4 *>(logits_out));
     return hipGetLastError();
 }
 

@@ -916,12 +916,9 @@ int Model::generate(int max_frames, const moss_hip_sample_params &p, uint64_t se
         if (timing) hip_check(hipEventRecord(ev[kEvLocal0], stream_), "event");
         launch_frame_local(stream_, gate_dump != nullptr, hstate_->cfg.greedy != 0);
         if (timing) hip_check(hipEventRecord(ev[kEvLocal1], stream_), "event");
-        if (logits_dump)
-            hip_check(hipMemcpyAsync(logits_h_ + (size_t)slot * kNVq * kCodebook, logits_,
-                                     sizeof(float) * kNVq * kCodebook, hipMemcpyDeviceToHost, stream_),
-                      "logits d2h");
-        hip_check(hipMemcpyAsync(hread_ + slot, state_, sizeof(DevState), hipMemcpyDeviceToHost, stream_),
-                  "state d2h");
+        hip_check(launch_frame_out(state_, hread_ + slot, logits_dump ? logits_ : nullptr,
+                                   logits_dump ? logits_h_ + (size_t)slot * kNVq * kCodebook : nullptr, stream_),
+                  "frame readback");
         hip_check(hipEventRecord(ev[kEvRead], stream_), "event");
         global_enq[slot] = f + 1 < max_frames && pos_next < max_ctx_;
         if (global_enq[slot]) {

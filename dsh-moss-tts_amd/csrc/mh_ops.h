@@ -382,6 +382,11 @@ hipError_t launch_copy_runs(const void *src, size_t src_stride, void *dst, size_
 // A row of 768 floats to host memory that the device can write (pinned): a 3 KB copy through
 // the runtime takes three times as long as this launch.
 hipError_t launch_row_out(const float *row, float *out, hipStream_t s);
+// A frame's decode state and, when logits is set, its [16][1024] logits, to pinned host memory.
+// The runtime's copies put the GPU through a system-wide fence before and after them: 23 us
+// a frame between its two halves, 10 with this launch.
+hipError_t launch_frame_out(const DevState *state, DevState *state_out, const float *logits, float *logits_out,
+                            hipStream_t s);
 // Device to device, every layer's K and V: positions [0, n_pos) of a contiguous cache
 // ([layer][head][ctx_stride][64], layer l of K at k_src + l * src_layer_elems) into the pages
 // of one stream (layer l of K at k_pool + l * pool_layer_elems), converted from src_kv to
