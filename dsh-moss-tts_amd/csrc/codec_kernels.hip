@@ -446,7 +446,10 @@ __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, 
 // 0.80 ms here, 1.13 before.
 template <int WV, bool XCD>
 __global__ __launch_bounds__(64 * WV) void codec_attn_kernel(const CodecAttnArgs a) {
-    __shared__ float red[WV][16 * 64 + 32];
+    // a wave's rows, 68 floats apart (16-byte reads and writes fall into different banks), then
+    // their maxima and sums
+    constexpr int kRow = kCodecHeadDim + 4, kStat = 16 * kRow;
+    __shared__ __align__(16) float red[WV][kStat + 32];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, col = lane & 15, grp = lane >> 4;
     int tile = blockIdx.x, h = blockIdx.y;
     if constexpr (XCD) {
@@ -557,31 +560,35 @@ __global__ __launch_bounds__(64 * WV) void codec_attn_kernel(const CodecAttnArgs
     }
     lrun += xshfl<16>(lrun);
     lrun += xshfl<32>(lrun);
-    // lane (grp, col) holds O[q col][16 grp + 4 i + j] = o[j][i]
+    // lane (grp, col) holds O[q col][16 grp + 4 i + j] = o[j][i]: rows of the head in LDS
     float *R = red[wave];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) R[(16 * grp + 4 * i + j) * 16 + col] = o[j][i];
+    for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4 *>(&R[col * kRow + 16 * grp + 4 * i]) = make_float4(o[0][i], o[1][i], o[2][i], o[3][i]);
     if (grp == 0) {
-        R[1024 + col] = mrun;
-        R[1040 + col] = lrun;
+        R[kStat + col] = mrun;
+        R[kStat + 16 + col] = lrun;
     }
     lds_barrier();
-    constexpr int E = 16 / WV;  // columns a thread finishes, of row t % 16
-    const int q = t & 15, d = E * (t >> 4), m = m0 + q;
+    constexpr int E = 16 / WV, TR = 64 / E;  // columns a thread finishes, threads a row
+    const int q = t / TR, d = E * (t % TR), m = m0 + q;
     if (m >= a.M) return;
     float mx = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < WV; ++w) mx = fmaxf(mx, red[w][1024 + q]);
+    for (int w = 0; w < WV; ++w) mx = fmaxf(mx, red[w][kStat + q]);
     const float msafe = mx == -INFINITY ? 0.f : mx;
     float l = 0.f, acc[E] = {};
 #pragma unroll
     for (int w = 0; w < WV; ++w) {
-        const float f = exp_f(red[w][1024 + q] - msafe);
-        l += f * red[w][1040 + q];
+        const float f = exp_f(red[w][kStat + q] - msafe);
+        l += f * red[w][kStat + 16 + q];
+        float r[E];
+        if constexpr (E == 4)
+            *reinterpret_cast<float4 *>(r) = *reinterpret_cast<const float4 *>(&red[w][q * kRow + d]);
+        else
+            *reinterpret_cast<float2 *>(r) = *reinterpret_cast<const float2 *>(&red[w][q * kRow + d]);
 #pragma unroll
-        for (int e = 0; e < E; ++e) acc[e] += f * red[w][(d + e) * 16 + q];
+        for (int e = 0; e < E; ++e) acc[e] += f * r[e];
     }
     if (a.splits == 1) {
         const float inv = 1.0f / l;

@@ -59,8 +59,9 @@ def test_w8a8_rows_do_not_depend_on_their_number(torch_gpu, rows, cols, m):
 @pytest.mark.parametrize("a16", [False, True])
 @pytest.mark.parametrize("kv32", [False, True])
 def test_long_prompt_is_its_pieces(torch_gpu, golden_model, a16, kv32):
-    """A prompt of 961 rows (its last tile holds one) in one call and 128 rows at a time (the
-    same fc_out split, no large tiles): the same keys, values and hidden state."""
+    """A prompt of 961 rows (its last tile holds one) in one call and in three of 352 and 353
+    (the same waves in the attention and the same fc_out split, no large tiles): the same keys,
+    values and hidden state."""
     print(f"a16={a16} kv32={kv32}", flush=True)
     blob, _ = golden_model
     n, rng = 961, np.random.default_rng(5)
@@ -71,9 +72,8 @@ def test_long_prompt_is_its_pieces(torch_gpu, golden_model, a16, kv32):
     m.prefill(rows)
     whole = (*m.kv_export(n), m.hidden())
     m.reset()
-    for at in range(0, n - 128, 128):  # 128 to 896, then the last 65 with 128 more before them
-        m.prefill(rows[at:at + 128], start=at)
-    m.prefill(rows[n - 129:], start=n - 129)
+    for at, end in ((0, 352), (352, 704), (608, n)):
+        m.prefill(rows[at:end], start=at)
     pieces = (*m.kv_export(n), m.hidden())
     m.close()
     for w, p in zip(whole, pieces):
