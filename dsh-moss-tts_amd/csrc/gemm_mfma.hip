@@ -377,7 +377,9 @@ __global__ __launch_bounds__(64 * WV, WV == 8 && EPI == EPI_RESID && NT == 2 ? 4
     constexpr bool kSplitFin = WV == 8 && NT >= 2;
     constexpr int FT = kSplitFin ? NT / 2 : NT;
     GT_START
-    __shared__ floatx4 red[WV][NT][64];
+    // the waves' partial sums, component i of every lane together: a finishing wave reads one
+    // component (of lane-wise vectors of 4, it met 4 lanes on a bank)
+    __shared__ float red[WV][NT][4][64];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int l16 = lane & 15, kq = lane >> 4;  // kq: which 8-column quarter of the block
     const int m_base = blockIdx.y * 16;
@@ -574,8 +576,10 @@ __global__ __launch_bounds__(64 * WV, WV == 8 && EPI == EPI_RESID && NT == 2 ? 4
         }
     }
 #pragma unroll
-    for (int t = 0; t < NT; ++t) red[wave][t][lane] = acc[t];
-    __syncthreads();
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[wave][t][i][lane] = acc[t][i];
+    lds_barrier();
     // lane holds rows m_base + 4kq + i, column n_base + 16t + l16
     if constexpr (EPI == EPI_GELU && NT >= 2 && WV == 4) {
         if (g.q8_out != nullptr) {  // uniform
@@ -583,13 +587,13 @@ __global__ __launch_bounds__(64 * WV, WV == 8 && EPI == EPI_RESID && NT == 2 ? 4
             // across the 16 lanes of a kq group, so its amax is a 16-lane reduction
             const int i = wave, m = erow;
             float h[NT];
-            const float *redf = (const float *)&red[0][0][lane] + i;
+            const float *redf = &red[0][0][i][lane];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                float v = redf[4 * (t * 64)];
-                v += redf[4 * ((NT + t) * 64)];
-                v += redf[4 * ((2 * NT + t) * 64)];
-                v += redf[4 * ((3 * NT + t) * 64)];
+                float v = redf[256 * t];
+                v += redf[256 * (NT + t)];
+                v += redf[256 * (2 * NT + t)];
+                v += redf[256 * (3 * NT + t)];
                 const int n = n_base + 16 * t + l16;
                 h[t] = gelu_new(v + eo.b[t]);
                 if (m < g.M && g.y != nullptr) g.y[(size_t)m * g.ldy + n] = h[t];
@@ -622,12 +626,12 @@ __global__ __launch_bounds__(64 * WV, WV == 8 && EPI == EPI_RESID && NT == 2 ? 4
     // component w of each lane's partials: one 4-byte LDS read each, at an offset
     // uniform in the wave; the waves' partials summed in wave order
     const int i = wave & 3, m = erow;
-    const float *redf = (const float *)&red[0][0][lane] + i;
+    const float *redf = &red[0][0][i][lane];
 #pragma unroll
     for (int t = 0; t < FT; ++t) {
-        float v = redf[4 * ((t0 + t) * 64)];
+        float v = redf[256 * (t0 + t)];
 #pragma unroll
-        for (int w = 1; w < WV; ++w) v += redf[4 * ((w * NT + t0 + t) * 64)];
+        for (int w = 1; w < WV; ++w) v += redf[256 * (w * NT + t0 + t)];
         const int n = n_base + 16 * (t0 + t) + l16;
         const float partner = xshfl<1>(v);  // column n ^ 1, same row
         if (m < g.M) gemm_finish<EPI, KV, FT>(er, eo, t, n, v, partner);
