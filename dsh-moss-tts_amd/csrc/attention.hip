@@ -412,8 +412,8 @@ __device__ __forceinline__ void tile_of_block(int block, int tiles, int &tile, i
 
 // Causal attention of 16 consecutive prompt rows x one head on the matrix cores (the
 // prefill: row r at position pos0 + r attends keys 0 .. pos0 + r of one cache page,
-// llm.cpp:349-392 over attention_core, llm.cpp:189-217).  Each of the WV waves takes every
-// WVth block of 16 keys with an online softmax, fp32 on v_mfma_f32_16x16x4_f32 (K/V widened
+// llm.cpp:349-392 over attention_core, llm.cpp:189-217).  Each of the 4 waves takes every
+// 4th block of 16 keys with an online softmax, fp32 on v_mfma_f32_16x16x4_f32 (K/V widened
 // from the cache's fp16 exactly):
 //   S^T = K Q^T: A = K[key kb + l%16][16g + t], B = Q[row l%16][16g + t], t = 0..15
 //   O^T = V^T P^T per column group j: A = V[key kb + 4g + s][4(l%16) + j], B = P[row][kb + 4g + s]
@@ -424,12 +424,13 @@ __device__ __forceinline__ void tile_of_block(int block, int tiles, int &tile, i
 // on the matrix cores (int8 under W8A8, fp16 hi / lo otherwise, the proj GEMM's per-block
 // arithmetic) and written as split-K partial h: one launch fewer per layer (the tile's
 // kernel time grows 9.7 -> 14.3 us against the 6.1 us proj GEMM it replaces).
-template <int KV, int WV>
-__global__ __launch_bounds__(64 * WV) void attn_tile_kernel(const AttnArgs a) {
+constexpr int kTileWaves = 4;
+template <int KV>
+__global__ __launch_bounds__(64 * kTileWaves) void attn_tile_kernel(const AttnArgs a) {
     // a wave's rows, 68 floats apart (16-byte reads and writes fall into different banks; as 64 columns
     // of 16 rows a merge read had 16 lanes on one bank, ~1 us a launch), then their maxima and sums
     constexpr int kRow = kHeadDim + 4, kStat = 16 * kRow;
-    __shared__ __align__(16) float red[WV][kStat + 32];
+    __shared__ __align__(16) float red[kTileWaves][kStat + 32];
     int tile, h;
     tile_of_block(blockIdx.x, (a.rows + 15) / 16, tile, h);
     if (tile < 0) return;  // uniform
@@ -544,21 +545,21 @@ __global__ __launch_bounds__(64 * WV) void attn_tile_kernel(const AttnArgs a) {
     float k0[16], k1[16];
     float4 v0[4], v1[4];
     if (wave < nkb) load_block(wave, k0, v0);
-    for (int b = wave; b < nkb; b += 2 * WV) {
-        load_block(b + WV, k1, v1);
+    for (int b = wave; b < nkb; b += 2 * kTileWaves) {
+        load_block(b + kTileWaves, k1, v1);
         block(b, k0, v0);
-        if (b + WV >= nkb) break;
-        load_block(b + 2 * WV, k0, v0);
-        block(b + WV, k1, v1);
+        if (b + kTileWaves >= nkb) break;
+        load_block(b + 2 * kTileWaves, k0, v0);
+        block(b + kTileWaves, k1, v1);
     }
     lrun += xshfl<16>(lrun);
     lrun += xshfl<32>(lrun);
-    // proj in the same launch (a.proj_part): wave w takes proj's 16-column subtiles w, w + WV,
+    // proj in the same launch (a.proj_part): wave w takes proj's 16-column subtiles w, w + kTileWaves,
     // ... of the 48; their units for this head's two blocks are requested now, so that they
     // arrive during the merge (the barriers up to the proj MFMAs order LDS only; requested
     // before the key blocks instead, they delay those: 256-row prefill 0.62 -> 0.63 ms)
     const bool fuse = a.proj_part != nullptr;  // uniform
-    constexpr int kPS = kHidden / 16 / WV;  // subtiles per wave
+    constexpr int kPS = kHidden / 16 / kTileWaves;  // subtiles per wave
     uint2 pq[kPS][2];
     uint16_t pd[kPS][2];
     if (fuse) {
@@ -571,7 +572,7 @@ __global__ __launch_bounds__(64 * WV) void attn_tile_kernel(const AttnArgs a) {
         for (int i = 0; i < kPS; ++i)
 #pragma unroll
             for (int bb = 0; bb < 2; ++bb) {
-                const int sub = wave + WV * i, blk = 2 * h + bb;
+                const int sub = wave + kTileWaves * i, blk = 2 * h + bb;
                 const uint8_t *qp, *dp;
                 if (a.proj_tiled) {
                     const uint8_t *unit = a.proj_w + ((size_t)sub * nb + blk) * kTileBytes;
@@ -596,17 +597,15 @@ __global__ __launch_bounds__(64 * WV) void attn_tile_kernel(const AttnArgs a) {
         R[kStat + 16 + col] = lrun;
     }
     lds_barrier();
-    // thread t < 256: row q = t / 16, columns 4 (t % 16) .. + 3 of the head (the waves past the
-    // fourth do the same work again and write nothing)
-    const bool fin = WV == 4 || t < 256;  // uniform over a wave
-    const int q = (t >> 4) & 15, d4 = t & 15, m = m0 + q;
+    // thread t: row q = t / 16, columns 4 (t % 16) .. + 3 of the head
+    const int q = t >> 4, d4 = t & 15, m = m0 + q;
     float mx = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < WV; ++w) mx = fmaxf(mx, red[w][kStat + q]);
+    for (int w = 0; w < kTileWaves; ++w) mx = fmaxf(mx, red[w][kStat + q]);
     const float msafe = mx == -INFINITY ? 0.f : mx;
     float l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < WV; ++w) {
+    for (int w = 0; w < kTileWaves; ++w) {
         const float f = expf(red[w][kStat + q] - msafe);
         const float4 r = *reinterpret_cast<const float4 *>(&red[w][q * kRow + 4 * d4]);
         l += f * red[w][kStat + 16 + q];
@@ -636,7 +635,7 @@ __global__ __launch_bounds__(64 * WV) void attn_tile_kernel(const AttnArgs a) {
             qq = qq < -127 ? -127 : (qq > 127 ? 127 : qq);
             qword |= (uint32_t)(qq & 0xff) << (8 * e);
         }
-        if (a.q8 != nullptr && m < a.rows && fin) {
+        if (a.q8 != nullptr && m < a.rows) {
             // 4 consecutive columns: one aligned 4-byte run of the matrix-core order
             *reinterpret_cast<uint32_t *>(a.q8 + q8t_at(m, h * kHeadDim + 4 * d4, kHidden)) = qword;
             if ((d4 & 7) == 0) a.d8[d8t_at(m, 2 * h + (d4 >> 3), kHidden)] = dq;
@@ -651,8 +650,7 @@ __global__ __launch_bounds__(64 * WV) void attn_tile_kernel(const AttnArgs a) {
         __shared__ float pda[2][16];
         __shared__ uint4 pah[2][64], pal[2][64];
         const int bb = d4 >> 3, L = q + 16 * ((d4 & 7) >> 1), half = d4 & 1;
-        if (!fin) {
-        } else if (a.proj_a8) {
+        if (a.proj_a8) {
             reinterpret_cast<uint32_t *>(&pa8[bb][L])[half] = qword;
             if ((d4 & 7) == 0) pda[bb][q] = dq;
         } else {
@@ -719,11 +717,11 @@ __global__ __launch_bounds__(64 * WV) void attn_tile_kernel(const AttnArgs a) {
             if (mr < a.rows) {
                 float *prow = a.proj_part + ((size_t)h * a.rows + mr) * kHidden + c16;
 #pragma unroll
-                for (int i = 0; i < kPS; ++i) prow[16 * (wave + WV * i)] = acc[i][r];
+                for (int i = 0; i < kPS; ++i) prow[16 * (wave + kTileWaves * i)] = acc[i][r];
             }
         }
     }
-    if (m >= a.rows || !fin) return;
+    if (m >= a.rows) return;
     if (a.out_hl != nullptr) {  // for the next GEMM: hi / lo halves in the matrix-core order
 #pragma unroll
         for (int e = 0; e < 4; ++e) store_hl(a.out_hl, m, h * kHeadDim + 4 * d4 + e, kHidden, ov[e]);
@@ -771,13 +769,10 @@ hipError_t launch_attn_tiles(const AttnArgs &a, KvType kv, hipStream_t s) {
     static_assert(kHeads == 12, "tile_of_block: 3 heads for 2 XCDs");
     const int tiles = (a.rows + 15) / 16;
     const dim3 grid(tiles_by_xcd(tiles) ? kXcds * tile_slots(tiles) : tiles * kHeads);
-    auto go = [&](auto kernel, int wv) { hipLaunchKernelGGL(kernel, grid, dim3(64 * wv), 0, s, a); };
-    // up to one workgroup per CU 8 waves share its keys and proj's columns (46, 181 rows, 29 rows
-    // after 181: 8.4, 11.4, 11.3 us a layer with 4, 8.0, 10.9, 10.6 with 8; 12 waves are slower than 4)
-    if (!tiles_by_xcd(tiles))
-        kv == KV_F16 ? go(attn_tile_kernel<KV_F16, 8>, 8) : go(attn_tile_kernel<KV_F32, 8>, 8);
+    if (kv == KV_F16)
+        hipLaunchKernelGGL(attn_tile_kernel<KV_F16>, grid, dim3(64 * kTileWaves), 0, s, a);
     else
-        kv == KV_F16 ? go(attn_tile_kernel<KV_F16, 4>, 4) : go(attn_tile_kernel<KV_F32, 4>, 4);
+        hipLaunchKernelGGL(attn_tile_kernel<KV_F32>, grid, dim3(64 * kTileWaves), 0, s, a);
     return hipGetLastError();
 }
 
