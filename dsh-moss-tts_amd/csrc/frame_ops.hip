@@ -374,6 +374,37 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const float *x, int x_s
     }
 }
 
+// The same, 4 values a thread, 8 lanes a 32-block, over all rows at once (quant_block32's
+// arithmetic): the row-per-workgroup kernel stores single bytes, 12 rounds of them one after the
+// other at K = 3072 (640 rows, quantised and
+// multiplied, 31.8 us; 27.4 with this).
+__global__ __launch_bounds__(256) void quant_rows4_kernel(const float *x, int x_stride, int K, size_t items, int8_t *q8,
+                                                          float *d8) {
+#pragma clang fp contract(off)
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= items) return;  // whole waves: K % 256 == 0
+    const int per = K / 4;
+    const size_t r = i / per;
+    const int c = 4 * (int)(i - r * per);
+    const float4 v = *reinterpret_cast<const float4 *>(x + r * x_stride + c);
+    float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+    amax = fmaxf(amax, xshfl<1>(amax));
+    amax = fmaxf(amax, xshfl<2>(amax));
+    amax = fmaxf(amax, xshfl<4>(amax));
+    const float d = amax / 127.0f;
+    const float id = d > 0.0f ? 1.0f / d : 0.0f;
+    const float e[4] = {v.x, v.y, v.z, v.w};
+    uint32_t w = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        int q = (int)rintf(e[k] * id);
+        q = q < -127 ? -127 : (q > 127 ? 127 : q);
+        w |= (uint32_t)(uint8_t)q << (8 * k);
+    }
+    *reinterpret_cast<uint32_t *>(q8 + r * K + c) = w;
+    if ((c & 31) == 0) d8[r * (K / 32) + (c >> 5)] = d;
+}
+
 // Split-K reduce + residual + LayerNorm of one row per workgroup (launch_resid_ln_rows).
 __global__ __launch_bounds__(256) void resid_ln_rows_kernel(const float *part, int ksplit, int rows,
                                                             const float *bias, const float *resid, int resid_stride,
@@ -871,6 +902,12 @@ hipError_t launch_quant_rows(const float *x, int x_stride, int K, int rows, int8
     if (rows <= 0) return hipSuccess;
     // every lane of a wave takes part in each block's shuffles: K a multiple of 256
     if (!x || !q8 || !d8 || K <= 0 || K % 256 != 0 || x_stride < K) return hipErrorInvalidValue;
+    const size_t items = (size_t)rows * (K / 4);
+    if ((uintptr_t)x % 16 == 0 && x_stride % 4 == 0 && (uintptr_t)q8 % 4 == 0 && items / 256 < INT32_MAX) {
+        hipLaunchKernelGGL(quant_rows4_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, x, x_stride, K, items,
+                           q8, d8);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(quant_rows_kernel, dim3(rows), dim3(256), 0, s, x, x_stride, K, q8, d8);
     return hipGetLastError();
 }

@@ -60,7 +60,7 @@ def test_w8a8_rows_do_not_depend_on_their_number(torch_gpu, rows, cols, m):
 @pytest.mark.parametrize("kv32", [False, True])
 def test_long_prompt_is_its_pieces(torch_gpu, golden_model, a16, kv32):
     """A prompt of 961 rows (its last tile holds one) in one call and in three of 352 and 353
-    (the same waves in the attention and the same fc_out split, no large tiles): the same keys,
+    (the same fc_out split, no large tiles): the same keys,
     values and hidden state."""
     print(f"a16={a16} kv32={kv32}", flush=True)
     blob, _ = golden_model
@@ -78,3 +78,24 @@ def test_long_prompt_is_its_pieces(torch_gpu, golden_model, a16, kv32):
     m.close()
     for w, p in zip(whole, pieces):
         assert np.array_equal(w, p)
+
+
+@pytest.mark.parametrize("m,cols", [(1, 256), (3, 768), (640, 3072)])
+def test_quantised_rows_do_not_depend_on_alignment(torch_gpu, m, cols):
+    """Rows that 16-byte loads and 4-byte stores may touch, and the same ones off by a value: the same
+    bytes and scales, with a block of zeros, of infinities and of NaN among them."""
+    torch = torch_gpu
+    x = torch.randn(m, cols, generator=torch.Generator("cuda").manual_seed(m), device="cuda")
+    x[0, 32:64] = 0.0
+    x[0, 70] = float("inf")
+    x[-1, 130] = float("nan")
+    odd = torch.empty(m * cols + 1, device="cuda")
+    odd[1:] = x.view(-1)
+    out = []
+    for src, off in ((x, 0), (odd[1:], 1)):
+        q = torch.empty(m * cols + off, device="cuda", dtype=torch.int8)
+        d = torch.empty(m, cols // 32, device="cuda")
+        lib.quantize_rows(src, m, cols, q[off:], d)
+        out.append((q[off:].clone(), d))
+    assert torch.equal(out[0][0], out[1][0])
+    assert torch.equal(out[0][1].nan_to_num(7.0), out[1][1].nan_to_num(7.0))
