@@ -21,7 +21,8 @@ cpu_baseline: the reference's own AVX2 CPU path (oracle/_ref, compiled from the
 reference sources) decoding the same frames from the same context-512 state on
 this host, at T = 4 threads (its published setting) and T = the CPU share of
 this process (physical cores, affinity, cgroup quota and OMP_NUM_THREADS,
-whichever is smallest); host_cpu reports lscpu's model, sockets and cores.
+whichever is smallest); null, like every cpu_ref below, where that library was
+never built (no reference checkout); host_cpu reports lscpu's model, sockets and cores.
 
 Also reported: the single GEMV (K = 768, N = 2304) replayed from a graph beside
 the reference's gemv_par; single-query decode attention (12 x 64 heads, fp16
@@ -453,7 +454,9 @@ def cpu_attention(reps: int = 20):
     """The reference's AVX2 single-query attention (attn_avx2.cpp:93, one thread) at the
     same context lengths: ctx - 1 cached keys plus the query row's own k/v."""
     sys.path.insert(0, os.path.join(ROOT, "oracle"))
-    from oracle import RefCpu
+    from oracle import REF_SO, RefCpu
+    if not os.path.exists(REF_SO):
+        return None
     r = RefCpu(a16_mode="decode")
     rng = np.random.default_rng(5)
     out = {}
@@ -560,8 +563,10 @@ def cpu_codec(blob, threads: int, chunks: int = 4):
     """The reference AudioDecoder (oracle/_ref) on the same protocol: the stream warmed
     past every window, then `chunks` chunks of 8 frames, `threads` threads."""
     sys.path.insert(0, os.path.join(ROOT, "oracle"))
-    from oracle import RefCpu, RefDecoder
+    from oracle import REF_SO, RefCpu, RefDecoder
     from mosship import codec_format as cf
+    if not os.path.exists(REF_SO):
+        return None
     rng = np.random.default_rng(5)
     d = RefDecoder(RefCpu(a16_mode="decode"), blob, threads=threads)
     try:
@@ -883,7 +888,7 @@ def main():
     cpu_st = {}
     if not args.no_cpu:
         share = host["cpu_share"]
-        log(f"cpu baseline (reference), share {share} cores")
+        log(f"cpu baseline (reference, if built here), share {share} cores")
         cpu = cpu_baseline(blob, state, args.steps, share)
         cpu_gv = cpu_gemv(share)
         cpu_at = cpu_attention()
