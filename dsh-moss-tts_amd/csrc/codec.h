@@ -95,16 +95,16 @@ int codec_advance_launch(int *pos0, const int *rows, hipStream_t s);  // pos0[i]
 
 // One stream's decoder state: per stage the next position and per layer the K/V rings.
 struct CodecState {
-    int *pos0 = nullptr;  // device [4]
+    uint8_t *mem = nullptr;  // holds all of it
+    int *pos0 = nullptr;     // device [4]
     int ring[kCodecStages] = {};
     std::vector<float *> k, v;  // per layer (all stages, in order), [ring_s][256] each
 };
 
-// The activations of one piece of at most `cap` frames.
+// The activations of one piece.
 struct CodecWork {
-    int cap = 0;
+    uint8_t *mem = nullptr;  // holds all of it
     int32_t *codes = nullptr;
-    size_t codes_cap = 0;
     float *z = nullptr, *xa = nullptr, *xb = nullptr, *y = nullptr, *qb = nullptr, *h = nullptr;
     float *ao = nullptr, *out = nullptr;
     float2 *ast = nullptr, *rope = nullptr;
@@ -144,8 +144,8 @@ private:
     void clear_state(CodecState &st);
     void alloc_work(CodecWork &w, int frames);
     void free_work(CodecWork &w);
-    void ensure_whole(int piece, int frames);
-    // launches of one piece of <= w.cap frames (codes on the device, `stride` apart per
+    void ensure_whole(int frames, int pieces);
+    // launches of one piece of no more frames than w was made for (codes on the device, `stride` apart per
     // quantizer), samples to w.out; stage_ev (5 events, [0] recorded by the caller) marks each
     // stage's end
     void enqueue(CodecState &st, CodecWork &w, const int32_t *codes, int stride, int frames, hipEvent_t *stage_ev);
@@ -154,7 +154,8 @@ private:
     void run_piece(CodecState &st, const int32_t *codes, int frames, float *out, bool graph);
 
     int device_ = 0;
-    int fmax_ = 32, spf_ = 0, ffn_max_ = 0;
+    int fmax_ = 32, whole_max_ = 0;  // frames of a piece: decode_chunk's, decode's
+    int spf_ = 0, ffn_max_ = 0;
     hipStream_t stream_ = nullptr;
     uint8_t *wdev_ = nullptr;  // every tensor of the file, 256-byte aligned
     const float *front_cb_[kCodecNq], *front_w_[kCodecNq], *front_b_[kCodecNq];
@@ -165,7 +166,9 @@ private:
     std::vector<LayerW> layers_;
     float *freq_ = nullptr;  // device [32]
     int c0_ = 0;             // q.out rows: the first stage's input width before its patch
-    CodecWork work_, whole_work_;
+    CodecWork work_, whole_work_;    // decode() has its own only if its pieces are longer than the stream's
+    int32_t *whole_codes_ = nullptr;  // decode(): the utterance's codes
+    size_t whole_codes_n_ = 0;
     int32_t *codes_host_ = nullptr;  // pinned staging
     float *out_host_ = nullptr;
     float *whole_host_[2] = {};      // decode(): the samples of two pieces, pinned

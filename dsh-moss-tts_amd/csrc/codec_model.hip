@@ -17,7 +17,8 @@ constexpr int kLayerCounts[kCodecStages] = {4, 2, 2, 4};    // decoder.cpp:44
 constexpr int kContexts[kCodecStages] = {500, 800, 1200, 1600};  // decoder.cpp:21
 constexpr int kDtF16 = 0, kDtF32 = 3;  // DType (csrc/include/moss/common.h:26)
 constexpr int kMaxPieceFrames = 1024;
-// decode() runs an utterance in equal pieces of at most this many frames
+// decode() runs an utterance in equal pieces of at most this many frames (of max_chunk_frames,
+// where the caller set it)
 constexpr int kWholePiece = 104;
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -35,6 +36,7 @@ Codec::Codec(const void *blob, size_t bytes, const moss_hip_codec_options &opt) 
     device_ = opt.device;
     fmax_ = opt.max_chunk_frames > 0 ? opt.max_chunk_frames : 32;
     if (fmax_ > kMaxPieceFrames) throw Status(MOSS_HIP_EINVAL, "max_chunk_frames > 1024");
+    whole_max_ = opt.max_chunk_frames > 0 ? fmax_ : kWholePiece;
     eager_ = opt.eager != 0;
     const uint8_t *b = static_cast<const uint8_t *>(blob);
     auto idx = parse_moss_index(b, bytes);
@@ -192,9 +194,9 @@ Codec::Codec(const void *blob, size_t bytes, const moss_hip_codec_options &opt) 
     hip_check(hipStreamSynchronize(stream_), "codec init");
 
     char buf[160];
-    std::snprintf(buf, sizeof(buf), "gpu decoder device=%d bytes=%zu ffn=%d windows=%d/%d/%d/%d pieces<=%d frames",
+    std::snprintf(buf, sizeof(buf), "gpu decoder device=%d bytes=%zu ffn=%d windows=%d/%d/%d/%d pieces<=%d frames, decode %d",
                   device_, arena, ffn_max_, stages_[0].window, stages_[1].window, stages_[2].window, stages_[3].window,
-                  fmax_);
+                  fmax_, whole_max_);
     info_ = buf;
 }
 
@@ -206,6 +208,7 @@ Codec::~Codec() {
     free_state(whole_state_);
     free_work(work_);
     free_work(whole_work_);
+    if (whole_codes_) (void)hipFree(whole_codes_);
     for (auto &set : ev_)
         for (auto &e : set)
             if (e) (void)hipEventDestroy(e);
@@ -231,6 +234,19 @@ int Codec::splits_for(int stage, int rows) const {
     return std::max(1, std::min(std::min(want, blocks / 16), kCodecMaxSplits));
 }
 
+namespace {
+// Parts of one allocation, each on a 256-byte boundary: what they take in all, then where they lie.
+struct Parts {
+    uint8_t *base = nullptr;
+    size_t bytes = 0;
+    template <class T>
+    void take(T *&p, size_t n) {
+        p = base ? reinterpret_cast<T *>(base + bytes) : nullptr;
+        bytes += align256(std::max<size_t>(n, 1) * sizeof(T));
+    }
+};
+}  // namespace
+
 // Buffers for pieces of up to `frames` frames.
 void Codec::alloc_work(CodecWork &w, int frames) {
     size_t xmax = (size_t)frames * c0_;  // q.out output = stage 0 input
@@ -243,82 +259,81 @@ void Codec::alloc_work(CodecWork &w, int frames) {
             part_rows = std::max(part_rows, (size_t)splits_for(s, r) * r);
         }
     for (int s = 0; s < kCodecStages; ++s) rope_rows += stage_rows(frames, s);
-    auto fmalloc = [&](float **p, size_t n) { hip_check(hipMalloc(p, std::max<size_t>(n, 64) * 4), "hipMalloc(codec act)"); };
-    w.codes_cap = (size_t)kCodecNq * frames;
-    hip_check(hipMalloc(&w.codes, sizeof(int32_t) * w.codes_cap), "hipMalloc(codes)");
-    fmalloc(&w.z, (size_t)frames * kCodecZ);
-    fmalloc(&w.xa, xmax);
-    fmalloc(&w.xb, xmax);
-    fmalloc(&w.y, rmax * kCodecDModel);
-    fmalloc(&w.qb, rmax * kCodecDModel);
-    fmalloc(&w.h, rmax * ffn_max_);
-    fmalloc(&w.ao, part_rows * kCodecDModel);
-    hip_check(hipMalloc(&w.ast, sizeof(float2) * part_rows * kCodecHeads), "hipMalloc(attn stats)");
-    hip_check(hipMalloc(&w.rope, sizeof(float2) * rope_rows * (kCodecHeadDim / 2)), "hipMalloc(rope)");
-    fmalloc(&w.out, (size_t)frames * spf_);
-    w.cap = frames;
+    auto parts = [&](uint8_t *base) {
+        Parts p{base};
+        p.take(w.codes, (size_t)kCodecNq * frames);
+        p.take(w.z, (size_t)frames * kCodecZ);
+        p.take(w.xa, xmax);
+        p.take(w.xb, xmax);
+        p.take(w.y, rmax * kCodecDModel);
+        p.take(w.qb, rmax * kCodecDModel);
+        p.take(w.h, rmax * ffn_max_);
+        p.take(w.ao, part_rows * kCodecDModel);
+        p.take(w.ast, part_rows * kCodecHeads);
+        p.take(w.rope, rope_rows * (kCodecHeadDim / 2));
+        p.take(w.out, (size_t)frames * spf_);
+        return p.bytes;
+    };
+    hip_check(hipMalloc(&w.mem, parts(nullptr)), "hipMalloc(codec activations)");
+    parts(w.mem);
 }
 
 void Codec::free_work(CodecWork &w) {
-    void *dev[] = {w.codes, w.z, w.xa, w.xb, w.y, w.qb, w.h, w.ao, w.ast, w.rope, w.out};
-    for (void *p : dev)
-        if (p) (void)hipFree(p);
+    if (w.mem) (void)hipFree(w.mem);
     w = CodecWork{};
 }
 
-// decode()'s own state and buffers, for pieces of `piece` frames of `frames`; they grow to the
-// largest piece asked for (at most kWholePiece frames) and are kept.
-void Codec::ensure_whole(int piece, int frames) {
-    if (piece > whole_work_.cap) {
-        hip_check(hipStreamSynchronize(stream_), "codec decode");
-        free_state(whole_state_);
-        free_work(whole_work_);
-        for (float *&p : whole_host_) {
-            if (p) (void)hipHostFree(p);
-            p = nullptr;
-        }
-        const int cap = std::min((piece + 31) / 32 * 32, kWholePiece);
-        alloc_state(whole_state_, cap);
-        for (float *&p : whole_host_)
-            hip_check(hipHostMalloc(&p, sizeof(float) * (size_t)cap * spf_), "hipHostMalloc(samples)");
-        alloc_work(whole_work_, cap);
-    }
+// What decode() keeps from its first call on: its state, its activations (the stream's serve where
+// the caller sized the pieces), pinned room for the samples of one piece, or two, and the codes of
+// the longest utterance so far.  All but the codes are made for the longest piece at once, one
+// allocation each: grown with the pieces asked for, ring by ring, a handle's utterances of 30, 40, 70
+// and 100 frames took 2.2, 2.9, 6.4 and 6.7 ms, now 0.8, 0.9, 1.2 and 1.4.
+void Codec::ensure_whole(int frames, int pieces) {
+    if (!whole_state_.mem) alloc_state(whole_state_, whole_max_);
+    if (whole_max_ != fmax_ && !whole_work_.mem) alloc_work(whole_work_, whole_max_);
+    for (int i = 0; i < std::min(pieces, 2); ++i)
+        if (!whole_host_[i])
+            hip_check(hipHostMalloc(&whole_host_[i], sizeof(float) * (size_t)whole_max_ * spf_), "hipHostMalloc(samples)");
     const size_t n = (size_t)kCodecNq * frames;
-    if (n > whole_work_.codes_cap) {
-        if (whole_work_.codes) hip_check(hipFree(whole_work_.codes), "free codes");
-        whole_work_.codes = nullptr;
-        whole_work_.codes_cap = 0;
-        hip_check(hipMalloc(&whole_work_.codes, sizeof(int32_t) * n), "hipMalloc(codes)");
-        whole_work_.codes_cap = n;
+    if (n > whole_codes_n_) {
+        if (whole_codes_) hip_check(hipFree(whole_codes_), "free codes");
+        whole_codes_ = nullptr;
+        whole_codes_n_ = 0;
+        const size_t room = (n + 16383) / 16384 * 16384;  // 1024 frames more at a time
+        hip_check(hipMalloc(&whole_codes_, sizeof(int32_t) * room), "hipMalloc(codes)");
+        whole_codes_n_ = room;
     }
 }
 
 // Rings for pieces of up to `frames` frames.
 void Codec::alloc_state(CodecState &st, int frames) {
-    hip_check(hipMalloc(&st.pos0, sizeof(int) * kCodecStages), "hipMalloc(codec pos)");
-    for (int s = 0; s < kCodecStages; ++s) {
-        st.ring[s] = stages_[s].window + stage_rows(frames, s);
-        for (int n = 0; n < stages_[s].nlayers; ++n) {
-            float *k = nullptr, *v = nullptr;
-            const size_t nb = sizeof(float) * st.ring[s] * kCodecDModel;
-            hip_check(hipMalloc(&k, nb), "hipMalloc(codec ring)");
-            hip_check(hipMalloc(&v, nb), "hipMalloc(codec ring)");
-            // zero once: a ring slot is only read after this stream wrote it, but keep it finite
-            hip_check(hipMemsetAsync(k, 0, nb, stream_), "clear ring");
-            hip_check(hipMemsetAsync(v, 0, nb, stream_), "clear ring");
-            st.k.push_back(k);
-            st.v.push_back(v);
+    auto parts = [&](uint8_t *base) {
+        Parts p{base};
+        p.take(st.pos0, kCodecStages);
+        st.k.clear();
+        st.v.clear();
+        for (int s = 0; s < kCodecStages; ++s) {
+            st.ring[s] = stages_[s].window + stage_rows(frames, s);
+            for (int n = 0; n < stages_[s].nlayers; ++n) {
+                float *k, *v;
+                p.take(k, (size_t)st.ring[s] * kCodecDModel);
+                p.take(v, (size_t)st.ring[s] * kCodecDModel);
+                st.k.push_back(k);
+                st.v.push_back(v);
+            }
         }
-    }
+        return p.bytes;
+    };
+    const size_t bytes = parts(nullptr);
+    hip_check(hipMalloc(&st.mem, bytes), "hipMalloc(codec rings)");
+    parts(st.mem);
+    // zero once: a ring slot is only read after this stream wrote it, but keep it finite
+    hip_check(hipMemsetAsync(st.mem, 0, bytes, stream_), "clear rings");
 }
 
 void Codec::free_state(CodecState &st) {
-    if (st.pos0) (void)hipFree(st.pos0);
-    for (float *p : st.k) (void)hipFree(p);
-    for (float *p : st.v) (void)hipFree(p);
-    st.pos0 = nullptr;
-    st.k.clear();
-    st.v.clear();
+    if (st.mem) (void)hipFree(st.mem);
+    st = CodecState{};
 }
 
 void Codec::clear_state(CodecState &st) {
@@ -555,10 +570,11 @@ void Codec::decode(const int32_t *codes, int frames, float *out) {
     // Equal pieces, each a long run of launches: while one computes, the host copies the samples
     // of the one before out of pinned memory.  (32-frame pieces, each waited for: 6.7 ms for 203
     // frames, a third of it launches too small for the chip and the copy.)
-    const int pieces = (frames + kWholePiece - 1) / kWholePiece, piece = (frames + pieces - 1) / pieces;
-    ensure_whole(piece, frames);
+    const int pieces = (frames + whole_max_ - 1) / whole_max_, piece = (frames + pieces - 1) / pieces;
+    ensure_whole(frames, pieces);
+    CodecWork &work = whole_work_.mem ? whole_work_ : work_;
     clear_state(whole_state_);
-    hip_check(hipMemcpyAsync(whole_work_.codes, codes, sizeof(int32_t) * kCodecNq * frames, hipMemcpyHostToDevice, stream_),
+    hip_check(hipMemcpyAsync(whole_codes_, codes, sizeof(int32_t) * kCodecNq * frames, hipMemcpyHostToDevice, stream_),
               "upload codes");
     double stage[kCodecStages] = {0, 0, 0, 0};
     auto finish = [&](int p) {  // the samples and stage times of piece p
@@ -574,8 +590,8 @@ void Codec::decode(const int32_t *codes, int frames, float *out) {
     for (int p = 0; p < pieces; ++p) {
         const int b = p & 1, f0 = p * piece, n = std::min(piece, frames - f0);
         hip_check(hipEventRecord(ev_[b][0], stream_), "hipEventRecord");
-        enqueue(whole_state_, whole_work_, whole_work_.codes + f0, frames, n, ev_[b]);
-        hip_check(hipMemcpyAsync(whole_host_[b], whole_work_.out, (size_t)n * spf_ * sizeof(float), hipMemcpyDeviceToHost,
+        enqueue(whole_state_, work, whole_codes_ + f0, frames, n, ev_[b]);
+        hip_check(hipMemcpyAsync(whole_host_[b], work.out, (size_t)n * spf_ * sizeof(float), hipMemcpyDeviceToHost,
                                  stream_),
                   "download samples");
         hip_check(hipEventRecord(done_[b], stream_), "hipEventRecord");

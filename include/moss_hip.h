@@ -346,9 +346,10 @@ typedef struct moss_hip_codec moss_hip_codec;
 
 typedef struct {
     int device;           /* HIP device ordinal */
-    int max_chunk_frames; /* a chunk is run in pieces of at most this many frames; 0 = 32.  Sizes the
-                             activation buffers and the K/V rings (window + 32 * this positions at the last
-                             stage).  Results do not depend on it beyond fp32 rounding. */
+    int max_chunk_frames; /* a chunk, and an utterance of decode(), is run in pieces of at most this many
+                             frames; 0 = 32, and 104 for decode().  Sizes the activation buffers and the K/V
+                             rings (window + 32 * this positions at the last stage).  Results do not depend
+                             on it beyond fp32 rounding. */
     int contexts[4];      /* per-stage attention windows in positions; 0 = the reference's 500, 800, 1200, 1600
                              (decoder.cpp:21; other values are for tests of the window) */
     int eager;            /* 0 = decode_chunk replays a hipGraph per piece size (default); 1 = direct launches */
@@ -369,7 +370,10 @@ int moss_hip_codec_reset_stream(moss_hip_codec *c);
  * frames * samples_per_frame floats.  Codes outside [0, 1024) -> EINVAL, nothing run. */
 int moss_hip_codec_decode_chunk(moss_hip_codec *c, const int32_t *codes, int frames, float *out);
 /* AudioDecoder::decode (decoder.cpp:247-281): a whole utterance from position 0, on a state
- * of its own (the stream is untouched); sets last_ms and the four stage times. */
+ * of its own (the stream is untouched); sets last_ms and the four stage times.  The first call
+ * allocates that state for the longest piece, which the handle keeps: 65 MB of rings at the default
+ * piece of 104 frames and windows, 27 MB at max_chunk_frames = 4; activations of its own (30 MB) only
+ * where max_chunk_frames is 0; and the codes, 64 bytes a frame of the longest utterance so far. */
 int moss_hip_codec_decode(moss_hip_codec *c, const int32_t *codes, int frames, float *out);
 double moss_hip_codec_last_ms(const moss_hip_codec *c);             /* decoder.h:31 */
 int moss_hip_codec_stage_ms(const moss_hip_codec *c, double out4[4]); /* decoder.h:32 */

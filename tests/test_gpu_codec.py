@@ -171,3 +171,40 @@ def test_codec_errors(torch_gpu, blob16, codec16):
     with pytest.raises(MossHipError) as e:
         HipCodec(bytes(broken))
     assert e.value.code == 4
+
+
+def _used(torch):
+    torch.cuda.synchronize()
+    free, total = torch.cuda.mem_get_info()
+    return total - free
+
+
+def test_decode_memory_follows_max_chunk_frames(torch_gpu, blob16, codec16):
+    """decode() runs in pieces of max_chunk_frames where the caller sets it, and holds rings for no
+    more (the activations are the stream's): 27 MB at 4 frames a piece, where pieces of 104 frames
+    took 126 MB.  8 MB of room for the codes and the allocator's pages."""
+    frames, piece = 512, 4
+    codes = _codes(frames, 21)
+    c = HipCodec(blob16, max_chunk_frames=piece)
+    c.decode_chunk(codes[:, :piece])
+    before = _used(torch_gpu)
+    y = c.decode(codes)
+    grown = _used(torch_gpu) - before
+    rows = np.cumprod(cf.PATCHES) * piece
+    rings = sum(n * 2 * (w + r) * cf.D_MODEL * 4 for n, w, r in zip(cf.LAYERS, cf.CONTEXTS, rows))
+    print(f"decode in pieces of {piece}: {grown / 1e6:.1f} MB, rings {rings / 1e6:.1f} MB", flush=True)
+    assert grown <= rings + (8 << 20)
+    c.close()
+    assert max_rel(y, codec16.decode(codes)) <= 1e-4
+
+
+def test_decode_allocates_once(torch_gpu, blob16):
+    """What decode() keeps is made by its first call, however short: longer utterances, of one piece
+    and of three, take no more (the codes, 64 bytes a frame, and one page of the allocator aside)."""
+    c = HipCodec(blob16)
+    c.decode(_codes(3, 1))
+    held = _used(torch_gpu)
+    for frames in (40, 70, 104, 211):
+        c.decode(_codes(frames, frames))
+        assert abs(_used(torch_gpu) - held) <= 2 << 20, frames
+    c.close()
