@@ -177,11 +177,11 @@ __global__ __launch_bounds__(256) void sample_kernel(SampleArgs a) {
     for (int c2 = t; c2 < kHidden; c2 += 256) a.next_input[c2] = q8x4_elem(a.aemb, nb, used, c2);
 }
 
-// grid (n_pos, layers, 2): position p of layer l of K (z = 0) or V (z = 1)
+// grid (n_pos, planes): position p of a plane, a layer's K or V
 template <int KV>
 __global__ __launch_bounds__(256) void kv_import_kernel(const float *src, int n_pos, void *dst, int ctx_stride) {
     const int p = blockIdx.x;
-    const size_t layer = blockIdx.z * gridDim.y + blockIdx.y;
+    const size_t layer = blockIdx.y;
     const float *row = src + (layer * n_pos + p) * kHidden;
 #pragma unroll
     for (int e = threadIdx.x; e < kHidden; e += 256) {
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) void kv_import_kernel(const float *src, int n_
 template <int KV>
 __global__ __launch_bounds__(256) void kv_export_kernel(const void *src, int n_pos, int ctx_stride, float *dst) {
     const int p = blockIdx.x;
-    const size_t layer = blockIdx.z * gridDim.y + blockIdx.y;
+    const size_t layer = blockIdx.y;
     float *row = dst + (layer * n_pos + p) * kHidden;
 #pragma unroll
     for (int e = threadIdx.x; e < kHidden; e += 256) {
@@ -270,27 +270,29 @@ hipError_t launch_sample(const SampleArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_kv_import(const float *src, int n_pos, void *kv_cache, int ctx_stride, KvType kv, hipStream_t s) {
+hipError_t launch_kv_import(const float *src, int n_pos, int planes, void *dst, int ctx_stride, KvType kv,
+                            hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
-    if (n_pos <= 0) return hipSuccess;
-    if (n_pos > ctx_stride) return hipErrorInvalidValue;
-    const dim3 grid(n_pos, kLayers, 2);
+    if (n_pos <= 0 || planes <= 0) return hipSuccess;
+    if (n_pos > ctx_stride || planes > 65535) return hipErrorInvalidValue;
+    const dim3 grid(n_pos, planes);
     if (kv == KV_F16)
-        hipLaunchKernelGGL(kv_import_kernel<KV_F16>, grid, dim3(256), 0, s, src, n_pos, kv_cache, ctx_stride);
+        hipLaunchKernelGGL(kv_import_kernel<KV_F16>, grid, dim3(256), 0, s, src, n_pos, dst, ctx_stride);
     else
-        hipLaunchKernelGGL(kv_import_kernel<KV_F32>, grid, dim3(256), 0, s, src, n_pos, kv_cache, ctx_stride);
+        hipLaunchKernelGGL(kv_import_kernel<KV_F32>, grid, dim3(256), 0, s, src, n_pos, dst, ctx_stride);
     return hipGetLastError();
 }
 
-hipError_t launch_kv_export(const void *kv_cache, int n_pos, int ctx_stride, KvType kv, float *dst, hipStream_t s) {
+hipError_t launch_kv_export(const void *src, int n_pos, int planes, int ctx_stride, KvType kv, float *dst,
+                            hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
-    if (n_pos <= 0) return hipSuccess;
-    if (n_pos > ctx_stride) return hipErrorInvalidValue;
-    const dim3 grid(n_pos, kLayers, 2);
+    if (n_pos <= 0 || planes <= 0) return hipSuccess;
+    if (n_pos > ctx_stride || planes > 65535) return hipErrorInvalidValue;
+    const dim3 grid(n_pos, planes);
     if (kv == KV_F16)
-        hipLaunchKernelGGL(kv_export_kernel<KV_F16>, grid, dim3(256), 0, s, kv_cache, n_pos, ctx_stride, dst);
+        hipLaunchKernelGGL(kv_export_kernel<KV_F16>, grid, dim3(256), 0, s, src, n_pos, ctx_stride, dst);
     else
-        hipLaunchKernelGGL(kv_export_kernel<KV_F32>, grid, dim3(256), 0, s, kv_cache, n_pos, ctx_stride, dst);
+        hipLaunchKernelGGL(kv_export_kernel<KV_F32>, grid, dim3(256), 0, s, src, n_pos, ctx_stride, dst);
     return hipGetLastError();
 }
 

@@ -9,6 +9,7 @@
 
 #include <array>
 #include <atomic>
+#include <functional>
 #include <stdexcept>
 #include <string>
 #include <unordered_map>
@@ -146,7 +147,7 @@ private:
     void launch_frame_local(hipStream_t s, bool text_gate, bool fused);
     void write_state_header();
     void *kv_layer(int which, int layer) const;  // which: 0 = K, 1 = V
-    float *kv_stage(int n_pos);
+    void kv_planes(int n_pos, const std::function<void(float *stage, int first, int n)> &move);
 
     int device_ = 0, max_ctx_ = kMaxCtx, use_graphs_ = 1;
     bool prefill_a16_ = false;  // prefill GEMMs on fp32 activations (else W8A8)
@@ -193,8 +194,8 @@ private:
     int rope_n_ = 0;
     float *hidden_h_ = nullptr;  // pinned: the hidden row on its way to the caller
     float *logits_h_ = nullptr;  // pinned: [2 readback slots][16][1024], when a caller takes logits
-    float *kv_stage_ = nullptr;  // kv_export / kv_import
-    size_t kv_stage_n_ = 0;      // its floats
+    float *kv_stage_ = nullptr;  // kv_export / kv_import: at most kKvStageKept bytes
+    size_t kv_stage_bytes_ = 0;
     float *x_ = nullptr, *q_ = nullptr, *mlp_ = nullptr, *hidden_ = nullptr;
     float *lres_ = nullptr, *next_in_ = nullptr, *slot_in_ = nullptr;
     float *attn_out_ = nullptr;

@@ -1053,40 +1053,75 @@ void Model::restore_prefix() {
     pos_ = prefix_pos_;
 }
 
-// The fp32 rows of n_pos positions of every layer's K and V, between kv_export / kv_import and
-// the caller's memory; grown to the largest call.
-float *Model::kv_stage(int n_pos) {
-    const size_t need = 2 * (size_t)kLayers * n_pos * kHidden;
-    if (need > kv_stage_n_) {
+// The fp32 rows of n_pos positions on their way between the cache and the caller's memory: `move`
+// takes planes first .. first + n - 1 of the cache's 24 (the layers' K, then their V) through
+// `stage`, as many at a time as 16 MiB hold (all of them up to 227 positions: one launch and two
+// copies where a launch, a copy and a wait for each took 1.13 ms for 46 positions, 0.65 now), but
+// at least one; one only on a device without room for more.  A stage up to that size is kept, a
+// larger one given back.
+constexpr size_t kKvStageKept = 16 << 20;
+
+void Model::kv_planes(int n_pos, const std::function<void(float *, int, int)> &move) {
+    const size_t plane = (size_t)n_pos * kHidden * 4;
+    int fit = (int)std::min<size_t>(std::max<size_t>(kKvStageKept / plane, 1), 2 * kLayers);
+    if (plane * fit > kv_stage_bytes_) {
         if (kv_stage_) hip_check(hipFree(kv_stage_), "free stage");
         kv_stage_ = nullptr;
-        kv_stage_n_ = 0;
-        hip_check(hipMalloc(&kv_stage_, need * 4), "hipMalloc(stage)");
-        kv_stage_n_ = need;
+        kv_stage_bytes_ = 0;
+        hipError_t e = hipMalloc(&kv_stage_, plane * fit);
+        if (e == hipErrorOutOfMemory && fit > 1) {
+            (void)hipGetLastError();
+            fit = 1;
+            e = hipMalloc(&kv_stage_, plane);
+        }
+        hip_check(e, "hipMalloc(stage)");
+        kv_stage_bytes_ = plane * fit;
     }
-    return kv_stage_;
+    struct GiveBack {
+        Model &m;
+        bool all;
+        ~GiveBack() {
+            if (!all) return;
+            (void)hipFree(m.kv_stage_);
+            m.kv_stage_ = nullptr;
+            m.kv_stage_bytes_ = 0;
+        }
+    } give_back{*this, kv_stage_bytes_ > kKvStageKept};
+    for (int p = 0; p < 2 * kLayers; p += fit) move(kv_stage_, p, std::min(fit, 2 * kLayers - p));
+    hip_check(hipStreamSynchronize(stream_), "sync");
+}
+
+// Planes first .. first + n - 1 of the caller's k and v, each [layer][n_pos][768]: `copy` gets
+// the run of them in k and the one in v, with its first plane's place in the stage.
+template <class P, class F>
+static void caller_runs(P *k, P *v, size_t plane, int first, int n, F &&copy) {
+    const int nk = std::max(0, std::min(n, kLayers - first));
+    if (nk > 0) copy(k + first * plane, (size_t)0, nk * plane);
+    if (n > nk) copy(v + (first + nk - kLayers) * plane, nk * plane, (n - nk) * plane);
 }
 
 void Model::kv_export(int n_pos, float *k, float *v) {
     if (n_pos < 0 || n_pos > max_ctx_) throw Status(MOSS_HIP_EINVAL, "n_pos out of range");
     if (n_pos == 0) return;
-    const size_t per = (size_t)kLayers * n_pos * kHidden;
-    float *stage = kv_stage(n_pos);
-    hip_check(launch_kv_export(kv_, n_pos, max_ctx_, kvt_, stage, stream_), "kv export");
-    hip_check(hipMemcpyAsync(k, stage, per * 4, hipMemcpyDeviceToHost, stream_), "kv d2h");
-    hip_check(hipMemcpyAsync(v, stage + per, per * 4, hipMemcpyDeviceToHost, stream_), "kv d2h");
-    hip_check(hipStreamSynchronize(stream_), "sync");
+    const size_t plane = (size_t)n_pos * kHidden;
+    kv_planes(n_pos, [&](float *stage, int first, int n) {
+        hip_check(launch_kv_export(kv_layer(0, first), n_pos, n, max_ctx_, kvt_, stage, stream_), "kv export");
+        caller_runs(k, v, plane, first, n, [&](float *to, size_t at, size_t len) {
+            hip_check(hipMemcpyAsync(to, stage + at, len * 4, hipMemcpyDeviceToHost, stream_), "kv d2h");
+        });
+    });
 }
 
 void Model::kv_import(int n_pos, const float *k, const float *v, const float *hidden) {
     if (n_pos < 0 || n_pos > max_ctx_) throw Status(MOSS_HIP_EINVAL, "n_pos out of range");
     if (n_pos > 0) {
-        const size_t per = (size_t)kLayers * n_pos * kHidden;
-        float *stage = kv_stage(n_pos);
-        hip_check(hipMemcpyAsync(stage, k, per * 4, hipMemcpyHostToDevice, stream_), "kv h2d");
-        hip_check(hipMemcpyAsync(stage + per, v, per * 4, hipMemcpyHostToDevice, stream_), "kv h2d");
-        hip_check(launch_kv_import(stage, n_pos, kv_, max_ctx_, kvt_, stream_), "kv import");
-        hip_check(hipStreamSynchronize(stream_), "sync");
+        const size_t plane = (size_t)n_pos * kHidden;
+        kv_planes(n_pos, [&](float *stage, int first, int n) {
+            caller_runs(k, v, plane, first, n, [&](const float *from, size_t at, size_t len) {
+                hip_check(hipMemcpyAsync(stage + at, from, len * 4, hipMemcpyHostToDevice, stream_), "kv h2d");
+            });
+            hip_check(launch_kv_import(stage, n_pos, n, kv_layer(0, first), max_ctx_, kvt_, stream_), "kv import");
+        });
     }
     if (hidden) set_hidden(hidden);
     pos_ = n_pos;

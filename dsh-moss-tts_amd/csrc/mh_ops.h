@@ -367,15 +367,17 @@ hipError_t launch_local_qkv_rows(const LocalQkv &a, int streams, hipStream_t s);
 // pos[s] += 1 for active streams; streams reaching capacity become inactive.
 hipError_t launch_advance_rows(const StreamState &st, int streams, hipStream_t s);
 
-// KV import/export of every layer between the reference layout, K then V as [layer][n][768]
-// fp32, and the device cache [K, V][layer][heads][ctx_stride][64] (fp16 or fp32).
-hipError_t launch_kv_import(const float *src, int n_pos, void *kv_cache, int ctx_stride, KvType kv, hipStream_t s);
+// KV import/export of consecutive planes (a layer's K or V) between the reference layout
+// [plane][n][768] fp32 and the device layout [plane][heads][ctx_stride][64] (fp16 or fp32).
+hipError_t launch_kv_import(const float *src, int n_pos, int planes, void *dst, int ctx_stride, KvType kv,
+                            hipStream_t s);
 // Same into pages: position p -> page table_row[p / page_size], slot p % page_size of [page][head][page_size][64].
 hipError_t launch_kv_import_paged(const float *src, int n_pos, void *pool, const int *table_row, int page_size,
                                   KvType kv, hipStream_t s);
 hipError_t launch_kv_export_paged(const void *pool, const int *table_row, int page_size, int n_pos, KvType kv,
                                   float *dst, hipStream_t s);
-hipError_t launch_kv_export(const void *kv_cache, int n_pos, int ctx_stride, KvType kv, float *dst, hipStream_t s);
+hipError_t launch_kv_export(const void *src, int n_pos, int planes, int ctx_stride, KvType kv, float *dst,
+                            hipStream_t s);
 // `runs` runs of `bytes`, each stride bytes after the one before (all multiples of 16).
 hipError_t launch_copy_runs(const void *src, size_t src_stride, void *dst, size_t dst_stride, size_t bytes, int runs,
                             hipStream_t s);

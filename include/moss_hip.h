@@ -152,7 +152,9 @@ int moss_hip_llm_restore_prefix(moss_hip_llm *m);
 int moss_hip_llm_prefix_pos(const moss_hip_llm *m);
 
 /* KV in the reference layout [12][n_pos][768] fp32 (llm.cpp:72-75), for the host
- * side of save_prefix / save_state (llm.cpp:485-586).  Export converts fp16 -> fp32. */
+ * side of save_prefix / save_state (llm.cpp:485-586).  Export converts fp16 -> fp32.  Both move
+ * the values through a staging buffer of up to 16 MiB that the handle keeps (a layer's K or V
+ * where that is larger, given back). */
 int moss_hip_llm_kv_export(moss_hip_llm *m, int n_pos, float *k, float *v);
 /* Import for load_prefix / load_state (llm.cpp:512-632): sets pos = n_pos and, when
  * hidden768 != NULL, the hidden state.  fp32 values are rounded to fp16 for an fp16 cache. */

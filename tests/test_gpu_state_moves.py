@@ -37,3 +37,28 @@ def test_state_moves(torch_gpu, golden_model, src32, dst32):
             assert all(np.array_equal(g, w) for g, w in zip(got, want))
     b.close()
     m.close()
+
+
+def test_moves_in_passes_keep_little(torch_gpu, golden_model):
+    """Import and export of more positions than the staging buffer holds at once: every layer's
+    K and V at the last size of one pass (227 positions), the first of two, five planes a pass and
+    one plane larger than the buffer.  What the model keeps afterwards is at most the buffer's 16 MiB
+    (and one page of the allocator)."""
+    blob, _ = golden_model
+    m = HipLLM(blob, max_ctx=5632)
+    rng = np.random.default_rng(4)
+
+    def used():
+        torch_gpu.cuda.synchronize()
+        free, total = torch_gpu.cuda.mem_get_info()
+        return total - free
+
+    start = used()
+    for n in (1, 227, 228, 1024, 5600):
+        print(f"n {n}", flush=True)
+        k, v = (rng.integers(-2048, 2049, (12, n, 768)).astype(np.float32) for _ in range(2))  # exact in fp16
+        m.kv_import(k, v, np.zeros(768, np.float32))
+        got = m.kv_export(n)
+        assert np.array_equal(got[0], k) and np.array_equal(got[1], v)
+        assert used() - start <= (16 << 20) + (2 << 20), n
+    m.close()
