@@ -152,8 +152,9 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
 #pragma unroll
         for (int i = 0; i < 3; ++i) act[t + 256 * i] = o[i];
         __syncthreads();
-        gate_block(act, a.wte, st, gl, SAMPLED ? gate_rng : st->rng);
-        // workgroup 0 changes the frame number and the stream only after the gate has read them
+        // no other workgroup waits for this one in a greedy frame, so by now workgroup 0 may have
+        // counted the frame in st->frame; a sampled frame's stream it stores after kLD only
+        gate_block(act, a.wte, st, gl, SAMPLED ? gate_rng : st->rng, a.frame);
         if constexpr (SAMPLED)
             if (t == 0) ll_put(LL + kLD, 1.0f, tag_base | 12u);
         return;

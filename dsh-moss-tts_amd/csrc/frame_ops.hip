@@ -82,7 +82,7 @@ __global__ __launch_bounds__(256) void gate_kernel(const float *x_raw, const flo
 #pragma unroll
     for (int i = 0; i < 3; ++i) hbuf[t + 256 * i] = o[i];
     __syncthreads();
-    gate_block(hbuf, wte, state, g, state->rng);
+    gate_block(hbuf, wte, state, g, state->rng, state->frame);
 }
 
 // End gate of a frame whose gate is dumped (llm.cpp:653-679): the reference then

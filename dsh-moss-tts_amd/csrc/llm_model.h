@@ -141,10 +141,10 @@ public:
 private:
     void enqueue_global_step(hipStream_t s, const int *row_dev);
     void enqueue_local_step(hipStream_t s, const float *in, int lpos, int pick_ch);
-    void enqueue_frame_local(hipStream_t s, bool text_gate, bool fused);
+    void enqueue_frame_local(hipStream_t s, int frame, bool text_gate, bool fused);
     void build_graphs();
     void launch_global(hipStream_t s);
-    void launch_frame_local(hipStream_t s, bool text_gate, bool fused);
+    void launch_frame_local(hipStream_t s, int frame, bool text_gate, bool fused);
     void write_state_header();
     void *kv_layer(int which, int layer) const;  // which: 0 = K, 1 = V
     void kv_planes(int n_pos, const std::function<void(float *stage, int first, int n)> &move);

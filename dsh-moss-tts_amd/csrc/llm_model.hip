@@ -455,7 +455,7 @@ void Model::enqueue_local_step(hipStream_t s, const float *in, int lpos, int pic
 // fused (greedy decoding): the pick of channel ch - 1 runs in the prologue of
 // channel ch's QKV GEMV instead of a kernel of its own; only channel 15 keeps
 // its sample kernel, which also counts the frame's used codes.
-void Model::enqueue_frame_local(hipStream_t s, bool text_gate, bool fused) {
+void Model::enqueue_frame_local(hipStream_t s, int frame, bool text_gate, bool fused) {
     if (fused_layers_ && !text_gate) {  // one launch
         LocalArgs c;
         const LayerW &L = local_;
@@ -484,6 +484,7 @@ void Model::enqueue_frame_local(hipStream_t s, bool text_gate, bool fused) {
         c.head = 1;
         c.gate = 1;
         c.wte = wte_;
+        c.frame = frame;
         c.final_pick = 1;
         c.sampled = fused ? 0 : 1;
         hip_check(launch_decode_local(c, s), "local steps");
@@ -536,7 +537,7 @@ void Model::build_graphs() {
     (void)hipGraphDestroy(g);
     for (int fused = 0; fused < 2; ++fused) {
         hip_check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
-        enqueue_frame_local(stream_, false, fused != 0);
+        enqueue_frame_local(stream_, 0, false, fused != 0);  // (per operator the frame's number is state->frame)
         hip_check(hipStreamEndCapture(stream_, &g), "end capture");
         hip_check(hipGraphInstantiate(fused ? &g_local_fused_ : &g_local_, g, nullptr, nullptr, 0),
                   "instantiate local");
@@ -551,12 +552,12 @@ void Model::launch_global(hipStream_t s) {
         enqueue_global_step(s, reinterpret_cast<const int *>(reinterpret_cast<uint8_t *>(state_) + kStateRowOff));
 }
 
-void Model::launch_frame_local(hipStream_t s, bool text_gate, bool fused) {
+void Model::launch_frame_local(hipStream_t s, int frame, bool text_gate, bool fused) {
     hipGraphExec_t g = fused ? g_local_fused_ : g_local_;
     if (g && !text_gate)
         hip_check(hipGraphLaunch(g, s), "graph launch");
     else
-        enqueue_frame_local(s, text_gate, fused);
+        enqueue_frame_local(s, frame, text_gate, fused);
 }
 
 // Pushes the scalar header (pos .. rep_penalty) of the host mirror to the device.
@@ -914,7 +915,7 @@ int Model::generate(int max_frames, const moss_hip_sample_params &p, uint64_t se
         const int slot = f & 1;
         hipEvent_t *ev = ev_ + kEvPerSlot * slot;
         if (timing) hip_check(hipEventRecord(ev[kEvLocal0], stream_), "event");
-        launch_frame_local(stream_, gate_dump != nullptr, hstate_->cfg.greedy != 0);
+        launch_frame_local(stream_, f, gate_dump != nullptr, hstate_->cfg.greedy != 0);
         if (timing) hip_check(hipEventRecord(ev[kEvLocal1], stream_), "event");
         hip_check(launch_frame_out(state_, hread_ + slot, logits_dump ? logits_ : nullptr,
                                    logits_dump ? logits_h_ + (size_t)slot * kNVq * kCodebook : nullptr, stream_),

@@ -456,15 +456,15 @@ __device__ __forceinline__ float gelu_new(float v) {
 // per-32-block activation quantisation (quant.cpp:28-54), the int32 block dots
 // of wte rows 7 (end) and 9 (slot) in the reference's lane order, the stop
 // rule.  Called by all 256 threads of a workgroup with h in LDS; thread 0
-// writes state->gate and, when the frame ends, state->stop; a sampled gate draws
-// from rng (thread 0's).
+// writes state->gate and, when frame `frame` ends the call, state->stop; a sampled
+// gate draws from rng (thread 0's).
 struct GateLds {
     int8_t qa[kHidden];
     float da[kHidden / 32];
     float lanes[2][8];
 };
 __device__ __forceinline__ void gate_block(const float *hbuf, const uint8_t *wte, DevState *state, GateLds &G,
-                                           uint32_t *rng) {
+                                           uint32_t *rng, int frame) {
 #pragma clang fp contract(off)
     const int t = threadIdx.x;
     int8_t *qa = G.qa;
@@ -516,7 +516,7 @@ __device__ __forceinline__ void gate_block(const float *hbuf, const uint8_t *wte
         }
         state->gate[0] = g[0];
         state->gate[1] = g[1];
-        if (state->frame >= state->min_frames && end_reached(g[1], g[0], state->cfg, rng)) state->stop = 1;
+        if (frame >= state->min_frames && end_reached(g[1], g[0], state->cfg, rng)) state->stop = 1;
     }
 }
 

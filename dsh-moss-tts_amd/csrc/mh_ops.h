@@ -465,6 +465,7 @@ struct LocalArgs {
     float *x_out = nullptr;            // block output (768)
     int gate = 0;                      // 1: after position 0, the W8A8 end gate (wte rows 7, 9); a stop ends the launch
     const uint8_t *wte = nullptr;
+    int frame = 0;                     // the frame's number (state->frame when the launch starts)
     int final_pick = 0;                // 1: after the last position, the pick of its channel, the
                                        // frame's code counts, row[0] = slot and frame + 1 (sample_kernel's work)
     int a8 = 0;                        // W8A8 GEMVs (activations quantised per 32-block), else W8A16

@@ -160,6 +160,33 @@ def test_generate_free_running_fp32kv(torch_gpu, oracle, prefilled):
     assert max_rel(g.hidden(), m.hidden()) <= TOL
 
 
+@pytest.mark.parametrize("greedy", [True, False])
+def test_min_frames_holds_the_gate_back(torch_gpu, oracle, greedy):
+    """The end gate of frame f counts from f = min_frames on, in the launch that also counts the
+    frame: the call ends at the frame where the oracle's does, for every min_frames (this model's
+    gate ends some frames and not others)."""
+    blob = mf.synth_model(10, ln_random=True)
+    rng = np.random.default_rng(0)
+    frames, rows = 8, mf.text_rows(rng.integers(0, mf.VOCAB, 20))
+    forced = np.full((frames, 17), mf.SLOT, np.int32)
+    forced[:, 1:] = rng.integers(0, 1024, (frames, 16))
+    m = oracle.model(blob)
+    m.prefill(rows, a16=True)
+    k, v, h = *m.kv_export(len(rows)), m.hidden()
+    lengths = []
+    g = HipLLM(blob, kv_fp32=True)
+    for n in range(frames + 1):
+        ref = _oracle_from_state(oracle, blob, k, v, h, kv_f16=False)
+        want = len(ref.generate(frames, OSP.make(greedy=True, min_frames=n), forced=forced)["rows"])
+        g.kv_import(k, v, h)
+        print(f"greedy {greedy} min_frames {n}: {want} frames", flush=True)
+        out = g.generate(frames, SampleParams.make(greedy=greedy, end_greedy=True, min_frames=n), forced=forced)
+        lengths.append(len(out["rows"]))
+        assert lengths[-1] == want >= n
+    g.close()
+    assert len(set(lengths)) > 3, lengths
+
+
 def test_generate_end_gate_matches_oracle(torch_gpu, oracle, prefilled):
     """min_frames = 0: the end gate decides when to stop.  Without a dump it is the
     2-row W8A8 gate; with a gate dump it is taken from the full text head, whose
