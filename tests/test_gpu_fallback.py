@@ -69,12 +69,12 @@ def test_waits_that_run_out_fall_back_to_per_operator(torch_gpu, state, monkeypa
     ref.close()
 
 
-@pytest.mark.parametrize("budget", ["1@1", "1@2", "1@3", "1@6", "3", "24"])
+@pytest.mark.parametrize("budget", ["1@0", "1@1", "1@2", "1@3", "1@5", "1@6", "3", "24"])
 def test_recovery_at_any_frame_matches_oracle(torch_gpu, oracle, state, monkeypatch, budget):
     """Waits that run out in a chosen launch ("1@K": one poll round from the model's K-th
-    fused launch on; launch 0 is the sampled local half captured into a graph at creation,
-    then generate alternates local half and global step: K = 1 hits L(0), 2 G(0) -- found
-    at frame 1's readback --, 3 L(1), 6 G(2)) or wherever a few poll rounds fall short
+    fused launch on; generate alternates local half and global step, and nothing before it
+    launches either: K = 0 hits L(0), 1 G(0) -- found at frame 1's readback --, 2 L(1), 3 G(1),
+    5 G(2), 6 L(3)) or wherever a few poll rounds fall short
     ("3", "24").
     Teacher-forced codes and logits against the oracle, and the final hidden state and
     position, to the usual bars."""
@@ -96,3 +96,56 @@ def test_recovery_at_any_frame_matches_oracle(torch_gpu, oracle, state, monkeypa
     assert max_rel(out["logits"], ref["logits"]) <= TOL
     assert max_rel(g.hidden(), m.hidden()) <= TOL and g.position == m.position
     g.close()
+
+
+SAMPLED = dict(greedy=False, temperature=0.9, top_p=0.95, repetition_penalty=1.3, end_greedy=False, min_frames=3)
+SAMPLED_BUDGETS = ["1@0", "1@1", "1@2", "1@5", "1@6"]
+
+
+@pytest.mark.parametrize("budget", SAMPLED_BUDGETS)
+@pytest.mark.parametrize("top_k", [40, 200])
+def test_recovery_of_a_sampled_call(torch_gpu, state, monkeypatch, budget, top_k):
+    """The same for a call that draws its codes and, from frame 3 on, its end: the draws go on per
+    operator from where the fused launches' stream stood, with the repetition counts of the frames
+    before, so codes and length are those of the per-operator model with the same seed.  (The
+    logits of the frames before the recovery differ in their last bits, which moves a draw only
+    within ~1e-6 of a boundary; none of these does.  Not under W8A8: there a last bit can become a
+    step of the int8 quantiser, 1 / 127 of a block's largest value, and the draws that land within
+    ~1e-2 of a boundary are many.)"""
+    blob, k, v, h = state
+    p = SampleParams.make(top_k=top_k, **SAMPLED)
+    ref = _model(blob, k, v, h, per_op=True)
+    want = ref.generate(8, p, seed=11)["rows"]
+    g = _model(blob, k, v, h, monkeypatch, budget=budget)
+    print(f"sampled generate, top_k {top_k}, budget {budget}, {len(want)} frames", flush=True)
+    got = g.generate(8, p, seed=11)["rows"]
+    assert g.fallbacks == 1
+    assert len(want) >= 3 and np.array_equal(got, want)
+    assert max_rel(g.hidden(), ref.hidden()) <= TOL and g.position == ref.position
+    g.close()
+    ref.close()
+
+
+@pytest.mark.parametrize("budget", SAMPLED_BUDGETS)
+@pytest.mark.parametrize("a8", [False, True])
+def test_recovered_draws_are_sample_tokens(torch_gpu, oracle, state, monkeypatch, budget, a8):
+    """Every draw before and after a recovery is sample_token's (sampler.cpp:9-79) on the logits that
+    it was made from (the call's own dump), the channel's history of forced codes and the call's
+    stream, in which the end gate draws before the codes from frame 3 on."""
+    blob, k, v, h = state
+    frames, seed, top_k = 6, 12, 40
+    forced = np.full((frames, 17), mf.SLOT, np.int32)
+    forced[:, 1:] = np.arange(16) * 61 % 1024  # the same codes: counts above one
+    g = _model(blob, k, v, h, monkeypatch, budget=budget, decode_a8=a8)
+    print(f"sampled generate, a8 {a8}, budget {budget}", flush=True)
+    out = g.generate(frames, SampleParams.make(top_k=top_k, **SAMPLED), seed=seed, forced=forced, logits=True)
+    assert g.fallbacks == 1 and len(out["rows"]) >= 3
+    g.close()
+    skip = 0
+    for f in range(len(out["rows"])):
+        skip += f >= SAMPLED["min_frames"]
+        for ch in range(16):
+            want = oracle.sample_token(out["logits"][f, ch], OSP.make(top_k=top_k, **SAMPLED),
+                                       prev=[int(forced[0, ch + 1])] * f, seed=seed, skip=skip)
+            skip += 1
+            assert out["rows"][f, ch + 1] == want, (f, ch)
