@@ -12,7 +12,7 @@ from conftest import max_rel
 import codec_oracle as co
 from mosship import HipCodec, MossHipError
 from mosship import codec_format as cf
-from mosship.moss_format import DT_F16, DT_F32, read_moss_index
+from mosship.moss_format import DT_F16, DT_F32, read_moss_index, write_moss
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-3
@@ -207,4 +207,53 @@ def test_decode_allocates_once(torch_gpu, blob16):
     for frames in (40, 70, 104, 211):
         c.decode(_codes(frames, frames))
         assert abs(_used(torch_gpu) - held) <= 2 << 20, frames
+    c.close()
+
+
+def test_decode_of_three_pieces(torch_gpu, blob16, codec16):
+    """From the third piece on decode() reuses its two sets of sample buffers and events, and a later
+    call its codes, rings and activations: 211 frames (71, 71 and 69) against the same codes
+    streamed, then a short utterance and a longer one (four pieces) on the same handle, then the
+    first again, which has to be the same bits.  (1e-4: two orders of the same fp32 sums.)"""
+    c = HipCodec(blob16)
+    first = None
+    for frames in (211, 5, 320, 211):
+        codes = _codes(frames, frames)
+        y = c.decode(codes)
+        codec16.reset_stream()
+        err = max_rel(y, codec16.decode_chunk(codes))
+        print(f"decode {frames} frames against the stream: max_rel {err:.2e}", flush=True)
+        assert err <= 1e-4
+        if frames == 211:
+            assert first is None or np.array_equal(y, first)
+            first = y
+    c.close()
+
+
+def test_decode_of_many_pieces_small_windows(torch_gpu, blob16, w16):
+    """22 frames in 6 pieces (max_chunk_frames 4) with windows of 8 to 20 positions: every ring wraps
+    within each piece."""
+    ctx = (8, 12, 16, 20)
+    codes = _codes(22, 8)
+    c = HipCodec(blob16, max_chunk_frames=4, contexts=ctx)
+    assert max_rel(c.decode(codes), co.Stream(w16, contexts=ctx).chunk(codes)) <= TOL
+    c.close()
+
+
+@pytest.mark.parametrize("frames", [9, 70, 104])
+def test_fp32_matrices_of_fp16_values(torch_gpu, blob16, codec16, frames):
+    """The same decoder with its matrices stored as fp32 (exactly the fp16 values): the same products,
+    through every tile size of the fp32-weight kernels (at 104 frames the last stage's all run in
+    64 x 64 tiles)."""
+    entries = []
+    for name, (dtype, rows, cols, off, n) in read_moss_index(blob16).items():
+        data = blob16[off:off + n]
+        if dtype == DT_F16:
+            dtype, data = DT_F32, np.frombuffer(data, np.float16).astype(np.float32).tobytes()
+        entries.append((name, dtype, rows, cols, data))
+    c = HipCodec(write_moss(entries))
+    codes = _codes(frames, 2 * frames)
+    err = max_rel(c.decode(codes), codec16.decode(codes))
+    print(f"fp32 matrices, {frames} frames: max_rel {err:.2e}", flush=True)
+    assert err <= 1e-6
     c.close()
