@@ -1,10 +1,10 @@
-// decode_local.hip -- one step of the local transformer of the single-stream decode in one launch (gfx950).
+// decode_local.hip -- a frame's local half of the single-stream decode in one launch (gfx950).
 //
-// Replaces local_step (reference csrc/src/llm.cpp:259-264: block_forward of the
-// one local layer at local position lpos, llm.cpp:230-246) and, for the
-// channel steps, the channel's audio head (audio_logits, llm.cpp:686-688:
-// logits = aemb[ch] . local_ln_f(x)).  The stages hand their outputs on through
-// LL words (mh_ll.h), as in decode_layer.hip:
+// Replaces the local steps of a frame (local_step, reference csrc/src/llm.cpp:259-264:
+// block_forward of the one local layer at local position lpos, llm.cpp:230-246),
+// the channels' audio heads (audio_logits, llm.cpp:686-688: logits = aemb[ch] .
+// local_ln_f(x)), the picks and the end gate.  Within each step lpos = 0 .. 16 the
+// stages hand their outputs on through LL words (mh_ll.h), as in decode_layer.hip:
 //   Q  lpos 0 only, b < 144: LN1 + QKV of the block input (the global hidden
 //      state), RoPE, k/v into the local cache                  -> LL q|k|v
 //   A  b < 12: head h = b: the step's input -- for lpos >= 2 the code of the
@@ -15,8 +15,8 @@
 //      0..lpos (at most 17)                                    -> LL attn + code
 //   P  b < 192: proj + residual (the raw input row is aemb[ch][code]) -> LL x + attn
 //   M  b < 192: LN2 + fc_in + gelu_new                          -> LL h
-//   F  b < 192: fc_out + residual -> x_out (memory) and, with a head, LL x_out
-//   H  b < 64, with a head: local ln_f + the audio head GEMV   -> logits (memory)
+//   F  b < 192: fc_out + residual -> x_out (memory) and, lpos >= 1, LL x_out
+//   H  b < 64, lpos >= 1: local ln_f + the audio head GEMV     -> logits (memory, LL)
 // (192 workgroups, one per CU; the GEMV stages take one wave per 4-row group,
 // or four for the K slices of proj and fc_out).
 //
@@ -34,7 +34,7 @@
 namespace mh {
 namespace {
 
-// LL regions (words); consecutive launches differ in lpos, so in tag
+// LL regions (words); consecutive steps differ in lpos, so in tag
 constexpr int kLQ = 0;                  // q | k | v (lpos 0)
 constexpr int kLA = kLQ + 3 * kHidden;  // attention output (768) and the step's input code (1)
 constexpr int kLX = kLA + kHidden + 1;  // x after the attention sub-block
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
     // ln_f of position 0's block output, the 2-row W8A8 gate, the stop rule.  The
     // channel steps do not wait for it: a frame the gate ends is dropped by the
     // host, and every state it touches is rewritten before it is read again.
-    if (a.gate && (int)blockIdx.x == kLayerGrid) {
+    if ((int)blockIdx.x == kLayerGrid) {
         const int t = threadIdx.x;
         float lw[3], lb[3];
 #pragma unroll
@@ -167,8 +167,13 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
         return idx >= kCodebook ? 0 : idx;  // every value NaN: the reference's scan stays at 0
     };
 
+    // positions 0 .. 16, the bounds hidden from the compiler: knowing them, it compiles a loop whose
+    // launch takes 219.5 us where one with the bounds as kernel arguments takes 217.5; this one takes
+    // 214.1 where that takes 214.8 (another card)
+    int first = 0, last = kNVq;
+    asm("" : "+s"(first), "+s"(last));
 #pragma unroll 1
-    for (int lpos = a.lpos; lpos <= a.lpos_last; ++lpos) {
+    for (int lpos = first; lpos <= last; ++lpos) {
         const int n = lpos + 1;
         const uint32_t tag = tag_base | (uint32_t)(12 + lpos);
         // per-step copies of the indices: nothing derived from them is held across steps
@@ -176,7 +181,7 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
         const int b = bix();
         const int ch_in = lpos >= 2 ? lpos - 2 : -1;  // channel whose code is this step's input
         const uint8_t *aemb_in = ch_in >= 0 ? a.aemb[ch_in] : nullptr;
-        const uint8_t *head_w = a.head && lpos >= 1 ? a.aemb[lpos - 1] : nullptr;
+        const uint8_t *head_w = lpos >= 1 ? a.aemb[lpos - 1] : nullptr;
         float *logits_out = lpos >= 1 ? a.logits + (size_t)(lpos - 1) * kCodebook : nullptr;
         const bool live = lpos == 0;  // the block input is the global hidden state: QKV computed here
         const bool picking = !live && ch_in >= 0;  // from the previous step's logits
@@ -239,7 +244,7 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
 #pragma unroll
                 for (int k = 0; k < kCodebook / 256; ++k)
                     pin.cnt[k] = st->rep_penalty != 1.0f ? a.counts[(size_t)ch_in * kCodebook + t + 256 * k] : 0;
-            // the cache rows (keys 0 .. lpos-1, written by earlier launches) before
+            // the cache rows (keys 0 .. lpos-1, written by earlier steps) before
             // anything else; the key at lpos, and the clamped ones past it, take
             // this step's row below
             float4 kr[kHeadDim / 4];
@@ -470,7 +475,7 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
                 if constexpr (A8)
                     if (cap) cap[MOSS_HIP_CAP_XOUT + r] = xo;
                 if (head_w) ll_put(LL + kLO + r, xo, tag);
-                if (live && a.gate) ll_put(LL + kLG + r, xo, tag);  // the gate workgroup's input
+                if (live) ll_put(LL + kLG + r, xo, tag);  // the gate workgroup's input
             }
             STAGE_TS(8);
             __syncthreads();
@@ -513,21 +518,21 @@ __global__ __launch_bounds__(256) void decode_local_kernel(LocalArgs a) {
             const float yv = gs.template dot<A8>(act, part, da);
             if (gs.storer()) {
                 logits_out[gs.row()] = yv;
-                if (lpos < a.lpos_last || a.final_pick) ll_put(LL + kLL + gs.row(), yv, tag);  // the next pick
+                ll_put(LL + kLL + gs.row(), yv, tag);  // the next pick
             }
             STAGE_TS(10);
         }
 
         // ---- after the last position: the pick of its channel, as
         // sample_kernel does for the last channel (workgroup 0)
-        if (a.final_pick && lpos == a.lpos_last && b == 0) {
+        if (lpos == last && b == 0) {
             const int ch = lpos - 1;
             PickIn pin;
 #pragma unroll
             for (int k = 0; k < kCodebook / 256; ++k)
                 pin.cnt[k] = st->rep_penalty != 1.0f ? a.counts[(size_t)ch * kCodebook + t + 256 * k] : 0;
             bool ok = ll_gather<kCodebook / 256>(LL + kLL, kCodebook, tag, lgt, budget);
-            if constexpr (SAMPLED) ok = ll_wait1(LL + kLD, t == 0 && a.gate, tag_base | 12u, &pbv[0], budget) && ok;
+            if constexpr (SAMPLED) ok = ll_wait1(LL + kLD, t == 0, tag_base | 12u, &pbv[0], budget) && ok;
             if (sync_failed(!ok, &wait_failed)) {
                 if (t == 0) atomicOr(a.err, 1u);
                 return;
@@ -576,20 +581,13 @@ hipError_t decode_local_occupancy(int *per_cu) {
 hipError_t launch_decode_local(const LocalArgs &a, hipStream_t s) {
     (void)hipGetLastError();  // report only this launch's error, not a stale one
     if (!a.attn_w || !a.proj_w || !a.fc_in_w || !a.fc_out_w || !a.lk || !a.lv || !a.state || !a.ll || !a.err ||
-        !a.x_out || a.lpos < 0 || a.lpos_last < a.lpos || a.lpos_last >= kLocalLen)
+        !a.x_out || !a.logits || !a.lnf_w || !a.lnf_b || !a.x_in || !a.rope_cos || !a.rope_sin || !a.wte ||
+        !a.qkv_table || !a.x_slot || !a.counts || !a.forced)
         return hipErrorInvalidValue;
-    if (a.head && (!a.logits || !a.lnf_w || !a.lnf_b)) return hipErrorInvalidValue;
-    for (int p = a.lpos < 1 ? 1 : a.lpos; p <= a.lpos_last; ++p)  // aemb rows: inputs (p >= 2) and heads
-        if ((p >= 2 && !a.aemb[p - 2]) || (a.head && !a.aemb[p - 1])) return hipErrorInvalidValue;
-    if (a.lpos == 0 && (!a.x_in || !a.rope_cos || !a.rope_sin)) return hipErrorInvalidValue;
-    if (a.gate && (a.lpos != 0 || !a.wte || !a.lnf_w || !a.lnf_b)) return hipErrorInvalidValue;
-    if (a.lpos_last >= 1 && !a.qkv_table) return hipErrorInvalidValue;
-    if (a.lpos <= 1 && a.lpos_last >= 1 && !a.x_slot) return hipErrorInvalidValue;
-    // a pick reads the logits of the launch's previous step: the steps run as one chain with heads
-    if (a.lpos_last >= 2 && (a.lpos > 1 || !a.head || !a.counts || !a.forced)) return hipErrorInvalidValue;
-    if (a.final_pick && (!a.head || a.lpos_last < 1 || !a.counts || !a.forced)) return hipErrorInvalidValue;
-    // one more workgroup for the end gate
-    const dim3 grid(kLayerGrid + (a.gate ? 1 : 0));
+    for (const uint8_t *w : a.aemb)
+        if (!w) return hipErrorInvalidValue;
+    static_assert(kNVq + 1 == kLocalLen, "positions 0 .. 16");
+    const dim3 grid(kLayerGrid + 1);  // one more workgroup for the end gate
     if (a.a8 && a.sampled)
         hipLaunchKernelGGL((decode_local_kernel<true, true>), grid, dim3(256), 0, s, a);
     else if (a.a8)

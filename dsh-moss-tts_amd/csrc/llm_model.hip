@@ -479,13 +479,8 @@ void Model::enqueue_frame_local(hipStream_t s, int frame, bool text_gate, bool f
         c.forced = forced_;
         c.x_in = hidden_;
         c.x_slot = slot_in_;
-        c.lpos = 0;  // positions 0..16, the gate and every channel's pick
-        c.lpos_last = kNVq;
-        c.head = 1;
-        c.gate = 1;
         c.wte = wte_;
         c.frame = frame;
-        c.final_pick = 1;
         c.sampled = fused ? 0 : 1;
         hip_check(launch_decode_local(c, s), "local steps");
         return;

@@ -440,7 +440,9 @@ struct GlobalArgs {
 };
 hipError_t launch_decode_global(const GlobalArgs &a, KvType kv, hipStream_t s);
 
-// ---- one local-transformer step (+ the channel's audio head) in one launch (decode_local.hip)
+// ---- a frame's local half in one launch (decode_local.hip): positions 0..16, the end gate after
+// position 0, the audio head of channel lpos - 1 after each later one, every channel's pick, and
+// with the last one the frame's code counts, row[0] = slot and frame + 1 (sample_kernel's work)
 struct LocalArgs {
     const uint8_t *attn_w = nullptr, *proj_w = nullptr, *fc_in_w = nullptr, *fc_out_w = nullptr;
     const float *attn_b = nullptr, *proj_b = nullptr, *fc_in_b = nullptr, *fc_out_b = nullptr;
@@ -451,23 +453,17 @@ struct LocalArgs {
     DevState *state = nullptr;
     uint64_t *ll = nullptr;
     unsigned *err = nullptr;
-    int lpos = 0;                      // first local position of the launch
-    int lpos_last = 0;                 // last one (positions 1..16 may run as one chain)
     const float *x_in = nullptr;       // lpos 0: block input (the global hidden state; QKV computed here)
     const float *x_slot = nullptr;     // lpos 1: the raw input row (dequantised wte[slot])
     const float *qkv_table = nullptr;  // [1 + 15 * 1024][2304]: row 0 for lpos 1, then (lpos, code) rows
     const uint8_t *aemb[kNVq] = {};    // audio embeddings / tied heads
     int sampled = 0;                   // 1: the call may draw its codes (state->cfg, state->rng), 0: greedy picks only
-    int head = 0;                      // 1: position lpos >= 1 also runs the audio head of channel lpos - 1
     float *logits = nullptr;           // [16][1024] head outputs (channel ch at ch * 1024)
     int *counts = nullptr;             // [16][1024] repetition counts (the final pick adds the frame's codes)
     const int *forced = nullptr;
     float *x_out = nullptr;            // block output (768)
-    int gate = 0;                      // 1: after position 0, the W8A8 end gate (wte rows 7, 9); a stop ends the launch
-    const uint8_t *wte = nullptr;
+    const uint8_t *wte = nullptr;      // the W8A8 end gate's rows 7 and 9
     int frame = 0;                     // the frame's number (state->frame when the launch starts)
-    int final_pick = 0;                // 1: after the last position, the pick of its channel, the
-                                       // frame's code counts, row[0] = slot and frame + 1 (sample_kernel's work)
     int a8 = 0;                        // W8A8 GEMVs (activations quantised per 32-block), else W8A16
     int poll_budget = 0;               // poll rounds a wait may take before it gives up (kPollBudget)
     float *cap = nullptr;              // W8A8 only: quantiser capture [kLocalLen][MOSS_HIP_CAP_STEP] (tests)
