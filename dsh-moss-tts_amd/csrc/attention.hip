@@ -386,13 +386,15 @@ __device__ __forceinline__ floatx4 mfma_f32x4(float a, float b, floatx4 c) {
 }
 
 // Workgroup -> (row tile, head) of the prefill attention.  Up to one workgroup per CU: every
-// head's tiles in order (all XCDs read all heads: at 256 rows 13.3 us a layer, 15.1 in the other
-// order, whose few XCDs per head all ask one L2 for the same lines).  Beyond: workgroups go to the
+// head's tiles in order (all XCDs read all heads: at 256 rows 12.3 us a layer, 13.2 in the other
+// order, whose few XCDs per head all ask one L2 for the same lines; at 336, 252 workgroups, 14.2 and
+// 15.1).  Beyond: workgroups go to the
 // 8 XCDs in turn and within one to its 32 CUs in turn, so an XCD works on its own head and half of
 // one that it shares with its neighbour, whose keys its L2 keeps, and its tiles go out in the order
 // of their length, every other round of 32 backwards: a CU that drew a long tile draws a short one
-// next (the last of 63 tiles has 63 times the keys of the first).  1000 rows 53.9 -> 36.9 us a
-// layer (fp32 keys 52.3 -> 36.0), 512 rows 25.6 -> 20.2, 384 rows 19.3 -> 17.5.
+// next (the last of 63 tiles has 63 times the keys of the first).  In order and so: 337 rows (264
+// workgroups) 16.2 and 14.7 us a layer, 384 17.5 and 15.5, 512 23.1 and 17.2, 1000 48.5 and 34.9 (fp32
+// keys 45.3 and 33.4).
 constexpr int kXcds = 8, kCusPerXcd = 32;
 __host__ __device__ constexpr bool tiles_by_xcd(int tiles) { return tiles * kHeads > kXcds * kCusPerXcd; }
 __host__ __device__ constexpr int tile_slots(int tiles) { return 3 * ((tiles + 1) / 2); }  // of one XCD

@@ -269,7 +269,7 @@ __global__ __launch_bounds__(256) void codec_gemm_kernel(const CodecGemmArgs g) 
 // different banks).  Consecutive workgroups go to different XCDs, so the tiles are numbered
 // such that all column tiles of a row tile run on one XCD and its L2 holds their rows.
 // (An utterance of 203 frames, with decode()'s long pieces: 6.66 ms in 32-frame pieces of 16 x 16
-// tiles, 3.30 ms.)
+// tiles, 2.75 ms now.)
 template <int PRO, int EPI, int WF32, int MT, int NT>
 __global__ __launch_bounds__(256) void codec_tile_kernel(const CodecGemmArgs g, int ntiles, int mtiles) {
     constexpr int kLdA = kCodecDModel + 4;
@@ -664,7 +664,16 @@ __global__ void codec_advance_kernel(int *pos0, Rows4 rows) {
     if (threadIdx.x < kCodecStages) pos0[threadIdx.x] += rows.r[threadIdx.x];
 }
 
-// Tiles of 64 x 64, or else 32 x 32, from this many of them on.
+// Tiles of 64 x 64, or else 32 x 32, from this many of them on: about one per CU, so that the chip
+// fills before a workgroup's own time grows.  Launches of one utterance in tiles of 16, 32 and 64 (us; N x K):
+//   768 x 256 (QKV):  224 rows 8.6, 6.7, 12.1; 352 11.6, 7.4, 12.1; 832 19.3, 10.2, 12.4;
+//                     1024 22.4, 10.4, 12.9; 1792 35.3, 16.7, 18.3; 3328 59.2, 26.3, 26.7
+//   1024 x 256 (f1):  224 rows 11.1, 7.0, 12.8; 640 19.3, 10.1, 13.4; 768 22.0, 10.2, 13.6; 3328 74.7, 32.3, 34.3
+//   256 x 1024 (f2):  1024 rows 14.2, 14.9, 29.3; 1152 16.6, 23.1, 29.4; 1664 21.8, 23.1, 29.5;
+//                     2560 29.9, 33.8, 29.9; 3328 37.6, 45.0, 30.4
+//   256 x 256 (proj): 896 rows 7.9, 7.8, 8.0; 1152 6.9, 7.8, 10.0; 1664 8.4, 8.0, 10.1; 2816 12.4, 10.5, 10.3
+// By them one line for all shapes is a compromise: 32 x 32 is already ahead at 120 tiles and still at
+// 1300 for the two wide products, and a long K does better in 16 x 16 until 64 x 64 fill the chip.
 constexpr long kTile64Min = 192, kTile32Min = 256;
 
 template <int PRO, int EPI, int MT, int NT>
@@ -727,7 +736,9 @@ int codec_attn_launch(const CodecAttnArgs &a, hipStream_t s) {
         return MOSS_HIP_EINVAL;
     const int tiles = (a.M + 15) / 16;
     static_assert(kCodecHeads == 4, "two XCDs a head");
-    if (a.splits == 1 && tiles * kCodecHeads > 256)  // more than one workgroup per CU
+    // more than one workgroup per CU: tiles by XCD and length, 4 waves (1024 rows, 256 workgroups: 17.2 us,
+    // 16.5 in order with 8 waves; 1152 rows 20.0 and 21.4, 1664 24.8 and 32.3, 3328 55.8 and 68.2)
+    if (a.splits == 1 && tiles * kCodecHeads > 256)
         hipLaunchKernelGGL((codec_attn_kernel<4, true>), dim3(8 * ((tiles + 1) / 2)), dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL((codec_attn_kernel<8, false>), dim3(tiles, kCodecHeads, a.splits), dim3(512), 0, s, a);

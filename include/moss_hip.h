@@ -373,8 +373,8 @@ int moss_hip_codec_reset_stream(moss_hip_codec *c);
 int moss_hip_codec_decode_chunk(moss_hip_codec *c, const int32_t *codes, int frames, float *out);
 /* AudioDecoder::decode (decoder.cpp:247-281): a whole utterance from position 0, on a state
  * of its own (the stream is untouched); sets last_ms and the four stage times.  The first call
- * allocates that state for the longest piece, which the handle keeps: 65 MB of rings at the default
- * piece of 104 frames and windows, 27 MB at max_chunk_frames = 4; activations of its own (30 MB) only
+ * allocates that state for the longest piece, which the handle keeps: 66 MB of rings at the default
+ * piece of 104 frames and windows, 27 MB at max_chunk_frames = 4; activations of its own (36 MB) only
  * where max_chunk_frames is 0; and the codes, 64 bytes a frame of the longest utterance so far. */
 int moss_hip_codec_decode(moss_hip_codec *c, const int32_t *codes, int frames, float *out);
 double moss_hip_codec_last_ms(const moss_hip_codec *c);             /* decoder.h:31 */
