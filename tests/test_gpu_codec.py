@@ -257,3 +257,11 @@ def test_fp32_matrices_of_fp16_values(torch_gpu, blob16, codec16, frames):
     print(f"fp32 matrices, {frames} frames: max_rel {err:.2e}", flush=True)
     assert err <= 1e-6
     c.close()
+
+
+def test_decode_in_one_long_piece(torch_gpu, blob16, codec16):
+    """max_chunk_frames beyond decode()'s own piece of 104: 211 frames in one, against three."""
+    c = HipCodec(blob16, max_chunk_frames=256)
+    codes = _codes(211, 211)
+    assert max_rel(c.decode(codes), codec16.decode(codes)) <= 1e-4
+    c.close()
