@@ -93,6 +93,41 @@ def test_batch_generate_vs_oracle(torch_gpu, oracle, setup):
     assert min(agree) >= 0.99
 
 
+@pytest.mark.parametrize("streams", [80, 81, 97, 193])
+def test_many_streams_vs_oracle(torch_gpu, oracle, setup, streams):
+    """The GEMMs of many rows: fc_out in 16-column tiles up to 80 streams and in 32-column tiles
+    beyond (81: the last row tile holds one stream), QKV and the heads in 64-column ones.  The streams
+    take the five states in turn: those of one state give the same bits, and each state's codes and
+    hidden state follow its oracle."""
+    blob, lens, states = setup
+    g = HipLLM(blob)
+    b = HipBatch(g, max_streams=streams, capacity=256, kv_fp32=True)
+    for s in range(streams):
+        b.set_stream(s, *states[s % len(states)])
+    frames = 3
+    print(f"{streams} streams", flush=True)
+    p = dict(greedy=True, min_frames=frames, repetition_penalty=1.2)
+    out = b.generate(streams, frames, SampleParams.make(**p))
+    assert (out["frames"] == frames).all()
+    agree = []
+    for j, (k, v, h) in enumerate(states):
+        hidden = b.hidden(j)
+        for s in range(j + len(states), streams, len(states)):
+            assert np.array_equal(out["rows"][:, s], out["rows"][:, j]) and np.array_equal(b.hidden(s), hidden), s
+        m = oracle.model(blob)
+        m.kv_import(k, v)
+        m.set_hidden(h)
+        forced = out["rows"][:, j].copy()
+        forced[:, 0] = mf.SLOT
+        eq = out["rows"][:, j, 1:] == m.generate(frames, OSP.make(**p), forced=forced)["rows"][:, 1:]
+        agree.append(float(np.mean(eq)))
+        if eq.all():
+            assert max_rel(hidden, m.hidden()) <= TOL
+    assert np.mean(agree) >= 0.99
+    b.close()
+    g.close()
+
+
 def test_batch_tiled_weights_bit_identical(torch_gpu, setup, monkeypatch):
     """The batch GEMMs (global layers, local layer, audio heads) read the matrices in the
     matrix-core order; with MOSS_HIP_GEMM_TILED=0 the Q8_0_4X4 ones: 3 sampled frames give
